@@ -999,6 +999,45 @@ def test_chunks_of_many_rows(gpu, d, Hkv, Hq, mapping):
     cache.close()
 
 
+@pytest.mark.parametrize("d,T", [(64, 28), (64, 40), (128, 28), (128, 40), (192, 28), (192, 40), (256, 28), (256, 40)])
+def test_merges_of_many_rows_by_rows_and_by_tiles(gpu, d, T):
+    """9 x 28 x 16 rows rotate by tiles and merge by rows, 9 x 40 x 16 rows do both by tiles, several partials a row:
+    every position as a call of that position alone gives it, into contiguous rows and a column-major tensor.  4e-6 per side,
+    as in test_chunks_of_many_rows."""
+    import torch
+    S, Hkv, Hq = 9, 4, 16
+    lens = [T, 41, 64, 65, 200, 333, 700, 40, 2500]
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(d + T)
+    cache = gpu.KVCache(gpu.KV_LLOYDMAX, S, Hkv, d, max(lens), 3, 4, 0, 0)
+    rk, rv = (torch.zeros(d * d, device="cuda") for _ in range(2))
+    gpu.make_rotation(5, d, rk)
+    gpu.make_rotation(6, d, rv)
+    cache.set_rotations(rk, rv)
+    for s, n in enumerate(lens):
+        k, v = (torch.randn((1, Hkv, n, d), generator=gen, device="cuda") for _ in range(2))
+        torch.cuda.synchronize()
+        cache.encode_append(k, v, seq_begin=s, rotate=1)
+        gpu.sync()
+    q = torch.randn((S, T, Hq, d), generator=gen, device="cuda")
+    flags = gpu.ATTN_ROTATE_Q | gpu.ATTN_UNROTATE_OUT
+    want = torch.zeros_like(q)
+    for t in range(T):
+        seen = torch.tensor([n - (T - 1 - t) for n in lens], dtype=torch.int32, device="cuda")
+        one, out1 = q[:, t].contiguous(), torch.zeros((S, Hq, d), device="cuda")
+        torch.cuda.synchronize()
+        cache.decode_attn_prefix(seen, one, out1, gqa_mapping=gpu.GQA_BLOCKED, flags=flags)
+        gpu.sync()
+        want[:, t] = out1
+    for out in (torch.zeros_like(q), torch.zeros((d, Hq, T, S), device="cuda").permute(3, 2, 1, 0)):
+        torch.cuda.synchronize()
+        cache.decode_attn_chunk(q, out, gqa_mapping=gpu.GQA_BLOCKED, flags=flags)
+        gpu.sync()
+        rel = float((out - want).double().norm() / want.double().norm())
+        assert rel <= 8e-6, (d, T, rel)
+    cache.close()
+
+
 def test_random_shapes_chunk_equals_single_positions(gpu):
     """Sixty seeded random shapes -- head_dim, coder, field widths, group size (also beyond a tile), chunk length,
     ragged lengths, GQA mapping: a chunk call must give what the single-position calls give (which the other tests

@@ -345,10 +345,10 @@ typedef float float16acc __attribute__((ext_vector_type(16)));
 // (v_mfma_f32_32x32x2f32).  Four wavefronts share the (row tile, column tile) pairs; a wavefront keeps its column tile's
 // part of M in registers for its row tiles.  The contraction index of an instruction may be any pair as long as both
 // operands agree: step i of eight k takes 8 i + 4 (lane / 32) + j in its instruction j, so that the rows come from LDS
-// in 16-byte pieces.  `first` holds the wavefront's first column tile's first KC / 2 elements (load_tile_columns).
+// in 16-byte pieces.  `b` comes with the wavefront's first column tile's first KC / 2 elements (load).
 template <int NT> struct TileRotation {
     static constexpr uint32_t D = 32 * NT, R = tile_rows_of(NT), PITCH = D + 4;
-    static constexpr uint32_t KC = NT % 4 == 0 ? 128 : (NT % 2 == 0 ? 64 : 32); // k per round of loads
+    static constexpr uint32_t KC = NT <= 4 ? D : D / 2;                         // k per round of loads
     static constexpr uint32_t CW = NT >= 4 ? 4 : (NT >= 2 ? 2 : 1);             // wavefronts side by side over the columns
     static constexpr uint32_t RW = 4 / CW;                                      // ... and over the row tiles
     static constexpr uint32_t RT = (R / 32 + RW - 1) / RW;                      // row tiles per wavefront
@@ -385,6 +385,13 @@ template <int NT> struct TileRotation {
                 for (uint32_t k0 = 0; k0 < D; k0 += KC) {
                     if (c || k0) {
                         load(b, m, ct, k0);
+                        // All of them requested before the first product: left alone, the compiler moves each load next to
+                        // the product that takes it, a trip to the second-level cache per instruction (a tile at head_dim
+                        // 96, 192 or 256 took 24, 43 or 53 us so, 8, 13 or 16 with the loads together).
+#pragma unroll
+                        for (uint32_t u = 0; u < KC / 2; ++u) {
+                            asm volatile("" : "+v"(b[u]));
+                        }
                     }
 #pragma unroll
                     for (uint32_t t = 0; t < RT; ++t) {
@@ -1117,26 +1124,39 @@ __global__ void __launch_bounds__(256) combine_tile_kernel(const float *__restri
     }
     __syncthreads();
     {
-        // weights: 256 / R lanes per row
-        constexpr uint32_t L = 256 / R;
+        // weights: 256 / R lanes per row, each slot's maximum and sum requested before the first is looked at
+        constexpr uint32_t L = 256 / R, U = 64 / L;
         const uint32_t r = tid / L, l = tid % L, n = n_s[r];
         const float *base = partials + (uint64_t)row_s[r] * max_slots * PS;
+        float2 t[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            if (u * L < max_slots) {
+                const uint32_t k = u * L + l;
+                t[u] = *reinterpret_cast<const float2 *>(base + (uint64_t)(k < n ? k : 0U) * PS);
+            }
+        }
         float mx = -INFINITY;
-        for (uint32_t k = l; k < n; k += L) {
-            const float m = base[(uint64_t)k * PS];
-            w_s[r][k] = m;
-            mx = fmaxf(mx, m);
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            if (u * L + l < n) {
+                mx = fmaxf(mx, t[u].x);
+            }
         }
 #pragma unroll
         for (uint32_t o = L / 2; o > 0; o >>= 1) {
             mx = fmaxf(mx, __shfl_xor(mx, (int)o));
         }
         float sum = 0.0f;
-        for (uint32_t k = l; k < n; k += L) {
-            const float m = w_s[r][k];
-            const float w = (m == -INFINITY) ? 0.0f : (log2_domain ? exp2f(m - mx) : expf(m - mx));
-            w_s[r][k] = w;
-            sum = fmaf(w, base[(uint64_t)k * PS + 1], sum);
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const uint32_t k = u * L + l;
+            if (k < n) {
+                const float m = t[u].x;
+                const float w = (m == -INFINITY) ? 0.0f : (log2_domain ? exp2f(m - mx) : expf(m - mx));
+                w_s[r][k] = w;
+                sum = fmaf(w, t[u].y, sum);
+            }
         }
 #pragma unroll
         for (uint32_t o = L / 2; o > 0; o >>= 1) {
@@ -1165,25 +1185,31 @@ __global__ void __launch_bounds__(256) combine_tile_kernel(const float *__restri
                     acc[i][c] = float2{ 0.0f, 0.0f };
                 }
             }
-            for (uint32_t k = 0; k < most; ++k) {
-                float2 v[2][NT];
-                float w[2];
+            constexpr uint32_t KU = NT <= 4 ? 4 : 2; // slots requested together
+            for (uint32_t k0 = 0; k0 < most; k0 += KU) {
+                float2 v[KU][2][NT];
 #pragma unroll
-                for (uint32_t i = 0; i < 2; ++i) {
-                    // (an unused slot may hold anything, so it is skipped rather than weighted with zero)
-                    w[i] = k < n[i] ? w_s[r0 + 16 * i + (tid >> 4)][k] : 0.0f;
+                for (uint32_t u = 0; u < KU; ++u) {
 #pragma unroll
-                    for (uint32_t c = 0; c < NT; ++c) {
-                        v[i][c] = w[i] != 0.0f ? *reinterpret_cast<const float2 *>(base[i] + (uint64_t)k * PS + 32 * c)
-                                               : float2{ 0.0f, 0.0f };
+                    for (uint32_t i = 0; i < 2; ++i) {
+                        const float *slot = base[i] + (uint64_t)(k0 + u < n[i] ? k0 + u : 0U) * PS;
+#pragma unroll
+                        for (uint32_t c = 0; c < NT; ++c) {
+                            v[u][i][c] = *reinterpret_cast<const float2 *>(slot + 32 * c);
+                        }
                     }
                 }
 #pragma unroll
-                for (uint32_t i = 0; i < 2; ++i) {
+                for (uint32_t u = 0; u < KU; ++u) {
 #pragma unroll
-                    for (uint32_t c = 0; c < NT; ++c) {
-                        acc[i][c].x = fmaf(w[i], v[i][c].x, acc[i][c].x);
-                        acc[i][c].y = fmaf(w[i], v[i][c].y, acc[i][c].y);
+                    for (uint32_t i = 0; i < 2; ++i) {
+                        // (an unused slot may hold anything, so it is skipped rather than weighted with zero)
+                        const float w = k0 + u < n[i] ? w_s[r0 + 16 * i + (tid >> 4)][k0 + u] : 0.0f;
+#pragma unroll
+                        for (uint32_t c = 0; c < NT; ++c) {
+                            acc[i][c].x = fmaf(w, w != 0.0f ? v[u][i][c].x : 0.0f, acc[i][c].x);
+                            acc[i][c].y = fmaf(w, w != 0.0f ? v[u][i][c].y : 0.0f, acc[i][c].y);
+                        }
                     }
                 }
             }
@@ -1238,8 +1264,14 @@ __global__ void __launch_bounds__(256) combine_tile_kernel(const float *__restri
     }
 }
 
-// From this many rows on the tiles fill the part (a tile is one workgroup's chain of gather, rotate, store).
+// From this many rows on the tiles of queries pay, at every head_dim and layout (4096 rows of 64, 96, 128, 192 or 256: 7.1,
+// 14.7, 10.6, 14.8 and 21.1 us by rows, 5.6, 8.4, 9.3, 12.6 and 15.2 in tiles; a tile is one workgroup's chain of gather,
+// rotate, store).  The merge's chain grows with the partials per row, half a microsecond each, while more rows shorten only
+// the row kernel's share: where there is one (head_dims that are multiples of 64) a merge of s partials goes by tiles from
+// 128 s rows more on (rows of 128: 4096 with 4, 9 or 25 partials 11.3, 12.1 and 16.6 us by rows, 12.6, 15.2 and 25.1 in
+// tiles; 6144 with 4 or 13: 17.6 and 22.8 against 12.6 and 19.8; rows of 256: 4096 with 25 partials 32.9 and 35.6).
 constexpr uint32_t kRowsForTiles = 4096;
+constexpr uint32_t kRowsPerPartialForTiles = 128;
 
 // The order in which the tiles walk a call's rows, and whether the rows' coordinates come in whole 16-byte pieces.  Rows
 // that are contiguous are taken in the order of their numbers; else the dimension with the smallest step in the caller's
@@ -1760,7 +1792,7 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
         ProfileScope prof("kv_decode_combine", timed);
         const SlotGeom sg = { use_mfma ? blk_off : nullptr, Hkv, G, runs,
                               gqa_mapping == WEED_HIP_GQA_BLOCKED ? 1 : 0, uniform_blocks };
-        if (tiles && n_splits <= 64) {
+        if (tiles && n_splits <= 64 && (d % 64 != 0 || n_rows >= kRowsForTiles + kRowsPerPartialForTiles * n_splits)) {
             int wide = 0;
             const RowOrder order = row_order(og, S, out_dev, d_real, wide);
             with_column_tiles(d, [&](auto nt) {
