@@ -1491,20 +1491,25 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
             }
         }
         // One workgroup per region instead, though that leaves compute units without one: its wavefronts' runs are longer,
-        // but the region is merged in the workgroup's LDS instead of through memory by the last of its workgroups (1.7 us,
-        // and up to 3.8 more with 256 workgroups arriving) or by runs that straddle regions (10 to 13 us).  A block
-        // more per wavefront is 1.7 us at 7 bits x 128 coordinates and goes by the block's bytes, 1.2 us at the least.
-        // Measured, 32 heads on 8 of 128: 16 sequences of 600-1000 tokens 19.0 -> 16.0 us, 1500 tokens 21.4 -> 17.7, 3000
-        // 23.7 -> 22.8, 4000 tokens 26.2 and 27.3 (stays); 24 sequences of 2000 tokens, whose runs straddled, 30.8 -> 20.2;
-        // 4 x 1000 tokens 16.3 -> 15.8, 1500 tokens 16.6 and 17.6 (stays).  12 heads of 64, one sequence of 1000 or 1500
-        // tokens: 11.9 and 12.2 -> 10.8; 8-bit fields, 4 x 1000 tokens: 18.6 and 19.5 (stays).
+        // but the region is merged in the workgroup's LDS instead of through memory by the last of its workgroups (2.6 us,
+        // and up to 2.9 more with 256 workgroups arriving) or by runs that straddle regions (10.5 us).  A block more per
+        // wavefront costs 1.7 us at 64 coordinates, 1.85 at 96, 2.6 at 128 and 3.3 above, a fifth less with uniform fields of
+        // up to 4 bits, twice as much where both sides look their codes up in tables of 32 (all from both plans' times of
+        // 500 drawn calls).
+        // 32 heads on 8 of 128: 16 sequences of 600-1000 tokens 19.0 -> 16.0 us, 24 of 2000, whose runs straddled, 30.8 ->
+        // 20.2; 12 heads of 64: one sequence of 1000 or 1500 tokens 11.9 and 12.2 -> 10.8.  Left as they are: 32 heads of
+        // 128 at 2 + 3 bits over 2174 tokens (16.6 us, 18.3 so), 48 heads of 64 with signs, 5 + 5 bits, over 3040-3424 (15.7
+        // and 21.4), 40 heads of 128 at 5 + 5 bits over 535 (17.4 and 19.1).
         if (!preferred_unit && may_round && (uint64_t)S * Hkv <= 256 &&
             mfma_decode_merges_whole_regions(pass_heads <= 4 ? 4u : (pass_heads <= 8 ? 8u : 16u), d, runs.waves)) {
             const uint32_t cand = (most + runs.waves - 1) / runs.waves * runs.waves, unit = cand / runs.waves;
             const uint32_t wg_blocks = runs.waves * runs.unit_blocks;
             const double wgs = std::min(256.0, std::ceil((double)total_blocks / wg_blocks));
-            const double merge_us = whole_shares ? 1.7 + 3.8 * wgs / 256.0 : 8.0;
-            const double block_us = std::max(1.2, 1.7 * (c->k.w + c->v.w) * d / 896.0);
+            const double merge_us = whole_shares ? 2.6 + 2.9 * wgs / 256.0 : 10.5;
+            const bool tables = c->cfg.mode == WEED_HIP_KV_LLOYDMAX;
+            const int wide_sides = (c->k.w > 4 ? 1 : 0) + (c->v.w > 4 ? 1 : 0);
+            const double block_us = (d <= 64 ? 1.7 : (d <= 96 ? 1.85 : (d <= 128 ? 2.6 : 3.3))) *
+                (tables ? 1.0 + 0.5 * wide_sides : 0.8 + 0.1 * wide_sides);
             if (cand <= reach && (uint64_t)cand * S * Hkv < (1ull << 32) &&
                 ((double)unit - runs.unit_blocks) * block_us < merge_us) {
                 virtual_blocks = cand == fewest ? 0 : cand;
