@@ -708,6 +708,31 @@ def test_dequant_of_contiguous_rows_equals_strided(gpu, d, w, tok_begin, T):
         cache.close()
 
 
+@pytest.mark.parametrize("S,Hkv,T", [(1, 1, 1), (3, 2, 64), (4, 16, 257), (16, 8, 256), (16, 8, 257)])
+def test_dequant_by_one_and_by_several_workgroups_per_block(gpu, S, Hkv, T):
+    """Calls of few blocks share each among up to eight workgroups, from 512 blocks on a workgroup takes a whole one: the
+    floats that the field-by-field path gives."""
+    import torch
+    d = 128
+    for mode in (gpu.KV_UNIFORM, gpu.KV_LLOYDMAX):
+        cache = gpu.KVCache(mode, S, Hkv, d, T, 4, 3)
+        if mode == gpu.KV_UNIFORM:
+            cache.set_scales(1.0, 0.8)
+        g = torch.Generator(device="cuda")
+        g.manual_seed(S * T)
+        x = [torch.randn((S, Hkv, T, d), generator=g, device="cuda") for _ in range(2)]
+        torch.cuda.synchronize()
+        cache.encode_append(x[0], x[1], rotate=0)
+        for which in (0, 1):
+            rows, strided = torch.zeros((S, Hkv, T, d), device="cuda"), torch.zeros((d, T, Hkv, S), device="cuda").permute(3, 2, 1, 0)
+            torch.cuda.synchronize()
+            cache.dequant(which, rows)
+            cache.dequant(which, strided)
+            gpu.sync()
+            assert torch.equal(rows, strided)
+        cache.close()
+
+
 @pytest.mark.parametrize("S,Hkv,d,lloyd", [(1, 1, 32, True), (3, 3, 64, False), (8, 8, 128, True), (5, 13, 128, False),
                                            (64, 8, 128, True), (57, 9, 96, True), (64, 16, 64, True), (41, 25, 128, True),
                                            (6, 2, 256, True), (3, 3, 80, False)])

@@ -989,14 +989,14 @@ __global__ void unpack_kernel(SideParams sp, int which, int kv_mode, uint32_t Hk
 // packed bytes come in once, 16 bytes per load, and the fields are picked out of LDS -- K: the four fields of a thread
 // are 4 w neighbouring bits; V: one field of each of four neighbouring items -- so that neighbouring lanes store
 // neighbouring 16-byte pieces of a row.  One byte load per field from memory and six integer divisions per float
-// (unpack_kernel) took 22 us for 4096 tokens x 8 heads x 128 at 3 bits, 0.8 TB/s; this takes 8.4
-// (2.0 TB/s; 4 us of any launch are its start and end).
+// (unpack_kernel) took 22 us for 4096 tokens x 8 heads x 128 at 3 bits, 0.8 TB/s; this takes 7.7
+// (2.2 TB/s; 4 us of any launch are its start and end).
 __global__ void __launch_bounds__(256) unpack_rows_kernel(SideParams sp, int which, int kv_mode, uint32_t Hkv, uint32_t d,
                                                           uint32_t d_stored, uint32_t padded, int32_t seq_begin,
                                                           uint32_t tok_begin, uint32_t T, float *__restrict__ out, Geom4 og)
 {
     __shared__ uint4 raw[kBlockTokens * 256 * 8 / 8 / 16 + 1]; // d_stored <= 256, w <= 8; one piece more: see `bits`
-    __shared__ float table[32];
+    __shared__ float table[32], alpha[kBlockTokens];
     const uint32_t h = blockIdx.y % Hkv, s = blockIdx.y / Hkv;
     const uint64_t region = (uint64_t)(seq_begin + (int32_t)s) * Hkv + h;
     const uint32_t block = tok_begin / kBlockTokens + blockIdx.x;
@@ -1005,17 +1005,21 @@ __global__ void __launch_bounds__(256) unpack_rows_kernel(SideParams sp, int whi
     for (uint32_t i = threadIdx.x; i < bytes / 16U; i += 256U) {
         raw[i] = src[i];
     }
+    const uint32_t first = max(tok_begin, block * kBlockTokens), last = min(tok_begin + T, (block + 1U) * kBlockTokens);
     if (threadIdx.x < 32) {
         table[threadIdx.x] = sp.table[threadIdx.x];
+    }
+    if (threadIdx.x < kBlockTokens) {
+        const uint32_t n = block * kBlockTokens + threadIdx.x; // (the region's scales cover whole blocks)
+        alpha[threadIdx.x] = sp.alpha ? sp.alpha[region * padded + n] : 0.0f;
     }
     __syncthreads();
     const uint32_t *words = reinterpret_cast<const uint32_t *>(raw);
     // up to 32 bits from any bit position on (the word behind the last one is read but its bits are not used)
     auto bits = [&](uint32_t at) { return __builtin_amdgcn_alignbit(words[at / 32U + 1U], words[at / 32U], at % 32U); };
     const uint32_t quads = d / 4U, w = sp.w, field_mask = (1U << w) - 1U;
-    const uint32_t first = max(tok_begin, block * kBlockTokens), last = min(tok_begin + T, (block + 1U) * kBlockTokens);
     float *dst = out + og.off + (uint64_t)s * og.s[0] + (uint64_t)h * og.s[1];
-    for (uint32_t i = threadIdx.x; i < (last - first) * quads; i += 256U) {
+    for (uint32_t i = blockIdx.z * 256U + threadIdx.x; i < (last - first) * quads; i += gridDim.z * 256U) {
         const uint32_t n = first + i / quads, j = i % quads * 4U;
         uint32_t f[4];
         if (which == 0) {
@@ -1033,7 +1037,7 @@ __global__ void __launch_bounds__(256) unpack_rows_kernel(SideParams sp, int whi
                 f[e] = bits(((uint32_t)p.byte + e * step) * 8U + p.bit) & field_mask;
             }
         }
-        const float a = sp.alpha ? sp.alpha[region * padded + n] : 0.0f;
+        const float a = alpha[n % kBlockTokens];
         float4 v;
         float *e4 = reinterpret_cast<float *>(&v);
 #pragma unroll
@@ -1403,7 +1407,13 @@ int launch_unpack(const weed_hip_kv_cache *c, int which, int32_t seq_begin, int3
                         ((reinterpret_cast<uintptr_t>(out_f) + 4ull * og.off) & 15U) == 0U;
     if (pieces && regions <= 65535U) {
         const uint32_t blocks = (uint32_t)(tok_begin + T - 1) / kBlockTokens - (uint32_t)tok_begin / kBlockTokens + 1U;
-        unpack_rows_kernel<<<dim3(blocks, (uint32_t)regions), 256, 0, stream()>>>(
+        // few blocks: each shared by up to eight workgroups, whose chains of pieces are that much shorter (64 tokens of 8 x 4
+        // heads of 256: 9.3 us by one workgroup per block, 4.9 so, which is a launch)
+        uint32_t slices = 1;
+        while (slices < 8U && blocks * regions * slices < 512U) {
+            slices *= 2U;
+        }
+        unpack_rows_kernel<<<dim3(blocks, (uint32_t)regions, slices), 256, 0, stream()>>>(
             sp, which, c->cfg.mode, (uint32_t)c->cfg.n_kv_heads, (uint32_t)c->cfg.head_dim, c->dp, c->padded_tokens,
             seq_begin, (uint32_t)tok_begin, (uint32_t)T, out_f, og);
         WEED_HIP_LAUNCH_CHECK();
