@@ -162,3 +162,46 @@ def test_short_products_in_a_graph_need_no_scratch(gpu, M, N, K):
         graph.replay()
         gpu.sync()
         assert bool(((out.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("warm", [False, True])
+def test_products_in_a_graph_outlive_the_scratch_they_were_captured_with(gpu, warm):
+    """Captured before the library has any scratch, products run without; captured after the same call has run, they use what
+    is there.  Either way the replays stay right after a larger product has taken a larger scratch: 17 to 64 rows on and off
+    the 16-byte grid, few whole and ragged tiles, k short and long."""
+    import torch
+    shapes = [(20, 600, 512), (32, 22001, 1025), (33, 2048, 2050), (64, 1024, 2048), (256, 512, 2048), (203, 301, 1030),
+              (40, 300, 4097)]
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(77)
+    gpu.shutdown()
+    gpu.check(gpu.load().weed_hip_init(0))
+    gpu.use_torch_stream(torch.cuda.current_stream())
+    work = []
+    for M, N, K in shapes:
+        a = torch.randn((K, M), generator=gen, device="cuda").t()
+        b = torch.randn((N, K), generator=gen, device="cuda").t()
+        out = torch.zeros((N, M), device="cuda").t()
+        bound = 4 * 1.2e-7 * (a.double().abs() @ b.double().abs())  # as the dense products' tests
+        work.append((a, b, out, a.double() @ b.double(), bound))
+    torch.cuda.synchronize()
+    if warm:
+        for a, b, out, _, _ in work:
+            gpu.matmul(a, b, out)
+        gpu.sync()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.current_stream()):
+        for a, b, out, _, _ in work:
+            gpu.matmul(a, b, out)
+    for i in range(4):
+        # 512 rows in up to 64 k ranges: more scratch than anything before, every pass another number of columns
+        N = 512 << i
+        big_a, big_b = torch.randn((16384, 512), generator=gen, device="cuda").t(), torch.randn((N, 16384), generator=gen, device="cuda").t()
+        big = torch.zeros((N, 512), device="cuda").t()
+        gpu.matmul(big_a, big_b, big)
+        for _, _, out, _, _ in work:
+            out.fill_(float("nan"))
+        graph.replay()
+        gpu.sync()
+        for (M, N, K), (_, _, out, want, bound) in zip(shapes, work):
+            assert bool(((out.double() - want).abs() <= bound).all()), (M, N, K, i)
