@@ -882,6 +882,47 @@ def test_infinities_off_the_sixteen_byte_grid(gpu, M, N, K):
     assert float(((out.double() - want).abs() / scale)[fine].max()) <= 4 * 1.2e-7
 
 
+@pytest.mark.parametrize("fp32_instruction", [False, True])
+@pytest.mark.parametrize("M,N,K", [(20, 513, 259), (33, 515, 1030), (131, 130, 127), (129, 127, 1031)])
+def test_tiny_and_huge_operands_off_the_sixteen_byte_grid(gpu, M, N, K, fp32_instruction):
+    """Off the 16-byte grid a product keeps what the fp32 instruction keeps, whichever instruction is asked for: operands
+    around 2^-120 and fp32 denormals against large ones, one tiny row or column among ordinary ones, the largest floats,
+    products that are denormals, infinities late in k.  The bound of the other products, plus half of the smallest denormal
+    per term where products get that small."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M * N + K)
+
+    def pair(a_scale, b_scale):
+        a = torch.randn((K, M), generator=gen, device="cuda", dtype=torch.float64) * a_scale
+        b = torch.randn((N, K), generator=gen, device="cuda", dtype=torch.float64) * b_scale
+        return a.float().t(), b.float().t()
+
+    cases = [pair(2.0 ** -120, 2.0 ** 120), pair(2.0 ** 100, 2.0 ** -138), pair(2.0 ** -70, 2.0 ** -60), pair(1, 1), pair(1, 1),
+             pair(2.0 ** -5, 2.0 ** -5)]
+    cases[3][0][5] *= 2.0 ** -125
+    cases[3][1].mul_(2.0 ** 90)
+    cases[4][1][:, 3] *= 2.0 ** -130
+    cases[5][0][2, 7] = 3.4028234e38
+    try:
+        gpu.matmul_tuning(fp32_instruction)
+        for i, (a, b) in enumerate(cases):
+            out = torch.zeros((N, M), device="cuda").t()
+            torch.cuda.synchronize()
+            gpu.matmul(a, b, out)
+            gpu.sync()
+            want, scale = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+            assert bool(((out.double() - want).abs() <= 4 * 1.2e-7 * scale + K * 2.0 ** -150).all()), i
+        a, b = pair(1, 1)
+        a[:, K - 2] = float("inf")
+        gpu.matmul(a, b, out)
+        gpu.sync()
+        want = a.double() @ b.double()
+        assert torch.equal(out.double(), want) and bool(out.isinf().all())
+    finally:
+        gpu.matmul_tuning(False)
+
+
 @pytest.mark.parametrize("M,N,K", [(128, 128, 272), (512, 512, 1296), (1024, 1024, 336), (1024, 1024, 752)])
 def test_whole_tiles_in_k_ranges_with_half_a_slice(gpu, M, N, K):
     """Whole 128 x 128 tiles whose K is an odd multiple of 16: the ranges may be whole 32-k slices, the last one is not.
