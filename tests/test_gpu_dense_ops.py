@@ -856,6 +856,30 @@ def test_products_off_the_sixteen_byte_grid(gpu, M, N, K):
                 assert err <= 4 * 1.2e-7, (a_rows, b_rows, gap, off, err)
 
 
+@pytest.mark.parametrize("fp32_instruction", [False, True])
+@pytest.mark.parametrize("M,N,K", [(17, 17, 2561), (32, 512, 2559), (32, 512, 2561), (32, 1023, 5121), (33, 40, 1281),
+                                   (64, 511, 1279), (64, 1024, 1281), (64, 2047, 3073), (17, 16, 4097)])
+def test_few_rows_and_columns_off_the_sixteen_byte_grid(gpu, M, N, K, fp32_instruction):
+    """Seventeen to 64 rows on both sides of where long k and few columns leave the streaming kernel for tiles in k ranges.
+    Bound as in test_split_k_partials_in_both_orders."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+    a = torch.randn((K, M), generator=gen, device="cuda").t()
+    b = torch.randn((N, K + 1), generator=gen, device="cuda")[:, :K].t()
+    bias = torch.randn((N,), generator=gen, device="cuda")
+    want, scale = a.double() @ b.double() + bias.double(), a.double().abs() @ b.double().abs() + bias.double().abs()
+    try:
+        gpu.matmul_tuning(fp32_instruction)
+        for out in (torch.zeros((N, M), device="cuda").t(), torch.zeros((M, N + 1), device="cuda")[:, :N]):
+            torch.cuda.synchronize()
+            gpu.linear(a, b, bias, out)
+            gpu.sync()
+            assert float(((out.double() - want).abs() / scale).max()) <= 4 * 1.2e-7
+    finally:
+        gpu.matmul_tuning(False)
+
+
 @pytest.mark.parametrize("M,N,K", [(20, 513, 259), (131, 130, 127), (129, 127, 1031)])
 def test_infinities_off_the_sixteen_byte_grid(gpu, M, N, K):
     """Infinite operands and ones next to the largest float where the split of an operand cannot take them: infinities of
@@ -883,7 +907,7 @@ def test_infinities_off_the_sixteen_byte_grid(gpu, M, N, K):
 
 
 @pytest.mark.parametrize("fp32_instruction", [False, True])
-@pytest.mark.parametrize("M,N,K", [(20, 513, 259), (33, 515, 1030), (131, 130, 127), (129, 127, 1031)])
+@pytest.mark.parametrize("M,N,K", [(20, 513, 259), (33, 515, 1030), (131, 130, 127), (129, 127, 1031), (64, 300, 4097)])
 def test_tiny_and_huge_operands_off_the_sixteen_byte_grid(gpu, M, N, K, fp32_instruction):
     """Off the 16-byte grid a product keeps what the fp32 instruction keeps, whichever instruction is asked for: operands
     around 2^-120 and fp32 denormals against large ones, one tiny row or column among ordinary ones, the largest floats,
