@@ -798,9 +798,9 @@ def test_norms_against_checker(gpu, oracle, shape, axis):
 @pytest.mark.parametrize("M,N,K", [(64, 1024, 2048), (33, 700, 1024), (200, 300, 2048), (203, 301, 1030), (130, 260, 4096)])
 def test_split_k_partials_in_both_orders(gpu, M, N, K):
     """Products whose k ranges go to several workgroups keep their partial sums in the order of the output: columns first,
-    rows first, off the 16-byte grid, with gaps and strided in both dimensions, with a bias; every element once.  The
-    same sums in the same order whatever the output's layout, and within 1.2e-7 of the terms' magnitudes per addition
-    chain (sqrt(K) of them at random signs) of float64."""
+    rows first, off the 16-byte grid, with gaps and strided in both dimensions, with a bias; every element once and nothing
+    between, before or behind them.  The same sums in the same order whatever the output's layout, bit for bit, and within
+    1.2e-7 of the terms' magnitudes per addition chain (sqrt(K) of them at random signs) of float64."""
     import torch
     gen = torch.Generator(device="cuda")
     gen.manual_seed(M + N)
@@ -818,9 +818,12 @@ def test_split_k_partials_in_both_orders(gpu, M, N, K):
         gpu.linear(a, w, bias, out)
         gpu.sync()
         assert float(((out.double() - want).abs() / scale).max()) <= 4 * 1.2e-7
-        assert bool((buf[:off] == 7.0).all()) and bool((buf[-8:] == 7.0).all())
-        outs.append(out.contiguous())
-    assert all(torch.equal(o, outs[0]) for o in outs[1:3])
+        outs.append(out.clone(memory_format=torch.contiguous_format))
+        out.fill_(7.0)
+        assert bool((buf == 7.0).all()), (stride, off)
+    # (outputs off the 16-byte grid of whole aligned operands go by instances of their own; the streamed products do not)
+    same = outs if M <= 64 else outs[:3]
+    assert all(torch.equal(o, outs[0]) for o in same[1:])
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 17, 257), (16, 130, 1027), (17, 600, 301), (64, 513, 258), (33, 515, 1030), (65, 33, 9),
