@@ -1190,6 +1190,9 @@ __global__ void __launch_bounds__(256) combine_tile_kernel(const float *__restri
                 float2 v[KU][2][NT];
 #pragma unroll
                 for (uint32_t u = 0; u < KU; ++u) {
+                    if (u && k0 + u >= most) {
+                        break;
+                    }
 #pragma unroll
                     for (uint32_t i = 0; i < 2; ++i) {
                         const float *slot = base[i] + (uint64_t)(k0 + u < n[i] ? k0 + u : 0U) * PS;
