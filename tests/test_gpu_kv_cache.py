@@ -708,9 +708,9 @@ def test_dequant_of_contiguous_rows_equals_strided(gpu, d, w, tok_begin, T):
         cache.close()
 
 
-@pytest.mark.parametrize("S,Hkv,T", [(1, 1, 1), (3, 2, 64), (4, 16, 257), (16, 8, 256), (16, 8, 257)])
+@pytest.mark.parametrize("S,Hkv,T", [(1, 1, 1), (3, 2, 8), (3, 2, 9), (3, 2, 64), (4, 16, 257), (16, 8, 256), (16, 8, 257)])
 def test_dequant_by_one_and_by_several_workgroups_per_block(gpu, S, Hkv, T):
-    """Calls of few blocks share each among up to eight workgroups, from 512 blocks on a workgroup takes a whole one: the
+    """Calls of few blocks share each among as many as eight workgroups, fewer than 9 rows of 128 or 512 blocks go without: the
     floats that the field-by-field path gives."""
     import torch
     d = 128

@@ -1002,17 +1002,20 @@ __global__ void __launch_bounds__(256) unpack_rows_kernel(SideParams sp, int whi
     const uint32_t block = tok_begin / kBlockTokens + blockIdx.x;
     const uint32_t bytes = block_bytes(d_stored, sp.w);
     const uint4 *src = reinterpret_cast<const uint4 *>(sp.fields + region * sp.region_bytes + (uint64_t)block * bytes);
+    // (levels and row scales requested with the block: one after the other, each a trip to memory of its own, reset + append +
+    // read back of 3 tokens took 36.5 us for 35.3 with the scales read per piece; the region's scales cover whole blocks)
+    const float level = sp.table[threadIdx.x % 32U];
+    const float scale = sp.alpha ? sp.alpha[region * padded + block * kBlockTokens + threadIdx.x % kBlockTokens] : 0.0f;
     for (uint32_t i = threadIdx.x; i < bytes / 16U; i += 256U) {
         raw[i] = src[i];
     }
-    const uint32_t first = max(tok_begin, block * kBlockTokens), last = min(tok_begin + T, (block + 1U) * kBlockTokens);
-    if (threadIdx.x < 32) {
-        table[threadIdx.x] = sp.table[threadIdx.x];
+    if (threadIdx.x < 32U) {
+        table[threadIdx.x] = level;
     }
     if (threadIdx.x < kBlockTokens) {
-        const uint32_t n = block * kBlockTokens + threadIdx.x; // (the region's scales cover whole blocks)
-        alpha[threadIdx.x] = sp.alpha ? sp.alpha[region * padded + n] : 0.0f;
+        alpha[threadIdx.x] = scale;
     }
+    const uint32_t first = max(tok_begin, block * kBlockTokens), last = min(tok_begin + T, (block + 1U) * kBlockTokens);
     __syncthreads();
     const uint32_t *words = reinterpret_cast<const uint32_t *>(raw);
     // up to 32 bits from any bit position on (the word behind the last one is read but its bits are not used)
@@ -1408,9 +1411,10 @@ int launch_unpack(const weed_hip_kv_cache *c, int which, int32_t seq_begin, int3
     if (pieces && regions <= 65535U) {
         const uint32_t blocks = (uint32_t)(tok_begin + T - 1) / kBlockTokens - (uint32_t)tok_begin / kBlockTokens + 1U;
         // few blocks: each shared by up to eight workgroups, whose chains of pieces are that much shorter (64 tokens of 8 x 4
-        // heads of 256: 9.3 us by one workgroup per block, 4.9 so, which is a launch)
+        // heads of 256: 9.3 us by one workgroup per block, 4.9 so, which is a launch), while every thread has a piece
         uint32_t slices = 1;
-        while (slices < 8U && blocks * regions * slices < 512U) {
+        const uint32_t block_pieces = std::min((uint32_t)T, kBlockTokens) * ((uint32_t)c->cfg.head_dim / 4U);
+        while (slices < 8U && blocks * regions * slices < 512U && slices * 256U < block_pieces) {
             slices *= 2U;
         }
         unpack_rows_kernel<<<dim3(blocks, (uint32_t)regions, slices), 256, 0, stream()>>>(
