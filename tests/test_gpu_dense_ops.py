@@ -969,3 +969,66 @@ def test_whole_tiles_in_k_ranges_with_half_a_slice(gpu, M, N, K):
         gpu.sync()
         scale = a.double().abs() @ b.double().abs()
         assert float(((out.double() - a.double() @ b.double()).abs() / scale).max()) <= 4 * 1.2e-7
+
+
+@pytest.mark.parametrize("M,N,K", [(128, 128, 96), (130, 133, 100), (132, 260, 2084), (256, 128, 12320)])
+@pytest.mark.parametrize("spread", ["even", "some", "fifth", "half", "late", "first", "zeros", "rows"])
+def test_products_of_halves_and_what_they_do_not_hold(gpu, M, N, K, spread):
+    """Split products keep the componentwise error of test_products_off_the_sixteen_byte_grid whatever the magnitudes: values
+    that half-precision parts of a tile's scale do not hold in no slice of k, in some, in every fifth (more than a workgroup
+    notes at 12320 k), in half of them, behind a first slice of another magnitude or of zeros; zeros among the values; rows of
+    very different magnitude in a tile.  Two products in one call (no k ranges), each with every layout of its operands.  Where
+    some terms are 2^60 and more times the others, a sum is hardly more than its largest term, rounded with every product that
+    follows: there the bound is that of test_matmul_random_shapes_through_the_dispatch."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+
+    def spread_out(x):  # [k, rows]
+        k = torch.arange(K, device="cuda")
+        some = {"some": k % 311 == 40, "fifth": k % 160 == 7, "half": k % 64 == 9}.get(spread)
+        if some is not None:
+            x[some] *= torch.exp2(torch.randint(-60, 61, (int(some.sum()), x.shape[1]), generator=gen, device="cuda").float())
+        elif spread == "late":
+            x[:40] *= 2.0 ** -40
+        elif spread == "first":
+            x[:32] = 0.0
+        elif spread == "zeros":
+            x[torch.rand(x.shape, generator=gen, device="cuda") < 0.4] = 0.0
+        elif spread == "rows":
+            x *= torch.exp2(torch.randint(-30, 31, (x.shape[1],), generator=gen, device="cuda").float())
+        return x
+
+    a_kr = torch.stack([spread_out(torch.randn((K, M), generator=gen, device="cuda")) for _ in range(2)])
+    b_kc = torch.stack([spread_out(torch.randn((K, N), generator=gen, device="cuda") * 0.02) for _ in range(2)])
+    bound = 2e-6 if spread in ("some", "fifth", "half") else 4 * 1.2e-7
+    want = a_kr.double().transpose(1, 2) @ b_kc.double()
+    scale = a_kr.double().abs().transpose(1, 2) @ b_kc.double().abs()
+    for a in (a_kr.transpose(1, 2), a_kr.transpose(1, 2).contiguous()):
+        for b in (b_kc, b_kc.transpose(1, 2).contiguous().transpose(1, 2)):
+            out = torch.zeros((2, N, M), device="cuda").transpose(1, 2)
+            torch.cuda.synchronize()
+            gpu.matmul_batched(a[None], b[None], out[None])
+            gpu.sync()
+            err = float(((out.double() - want).abs() / scale.clamp_min(1e-300)).max())
+            assert bool(out.isfinite().all()) and err <= bound, (a.stride(), b.stride(), err)
+
+
+@pytest.mark.parametrize("along_rows", [True, False])
+def test_products_with_long_strides(gpu, along_rows):
+    """Strides beyond the reach of the split-operand tiles' 32-bit offsets go by the fp32 instruction."""
+    import torch
+    M, N, K, stride = 20, 24, 40, (1 << 22) + 8
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(7)
+    slow = K if along_rows else M
+    base = torch.zeros((slow - 1) * stride + 64, device="cuda")
+    a = torch.as_strided(base, (M, K), (1, stride) if along_rows else (stride, 1))
+    a.copy_(torch.randn((M, K), generator=gen, device="cuda"))
+    b = torch.randn((N, K), generator=gen, device="cuda").t()
+    out = torch.zeros((N, M), device="cuda").t()
+    torch.cuda.synchronize()
+    gpu.matmul(a, b, out)
+    gpu.sync()
+    scale = a.double().abs() @ b.double().abs()
+    assert float(((out.double() - a.double() @ b.double()).abs() / scale).max()) <= 4 * 1.2e-7
