@@ -94,12 +94,12 @@ int weed_hip_matmul_f32(uint32_t M, uint32_t N, uint32_t K, const float *a_dev, 
  * one dimension (of 17 to 64 rows against a k-contiguous weight with 256 k or more: those of 512 columns or more, and
  * off the 16-byte grid those of a k too long for the streaming kernel) run on the 16-bit matrix instructions with both
  * operands split: as three products of half-precision parts (of 11 bits each, behind a power-of-two scale per tile of
- * the operand) where a slice of 32 k holds no values outside 2^-26 .. 2^2 of the largest in the tile's first slice, and
- * otherwise, as the products of 17 to 64 rows throughout, as six of the nine products of three exact bfloat16 parts;
- * accumulated in fp32 either way.  Twice the fp32 instruction's speed and more.  The error against the exact product is
+ * the operand) where a slice of 32 k holds no values above 2^6 of the largest in the tile's first 64 k and values below
+ * 2^-22 of it in one operand at most, and otherwise, as the products of 17 to 64 rows throughout, as six of the nine
+ * products of three exact bfloat16 parts; accumulated in fp32 either way.  Twice the fp32 instruction's speed and more.  The error against the exact product is
  * no larger than the fp32 instruction's own: 2.2e-7 of the result's norm for normal operands at k = 4096, 1.2e-7 at k =
  * 768 (5.0e-7 and 1.3e-7 as six products); relative to sum_k |a_ik| |b_kj| per element, for operands spanning
- * 2^-20 .. 2^20 at k = 1028, where every slice goes by six products, largest 7.1e-7 against 5.9e-7 and mean 5.8e-8
+ * 2^-20 .. 2^20 at k = 1028, where the slices go by six products, largest 7.1e-7 against 5.9e-7 and mean 5.8e-8
  * against 5.1e-8.  Two things the split does not keep: an operand that is not finite gives NaN where the fp32
  * instruction would give an infinity, and operand values below 2^-112 in magnitude lose accuracy where they go by
  * bfloat16 parts, because their second and third parts fall below bfloat16's normal range and the

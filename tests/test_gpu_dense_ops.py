@@ -972,13 +972,15 @@ def test_whole_tiles_in_k_ranges_with_half_a_slice(gpu, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(128, 128, 96), (130, 133, 100), (132, 260, 2084), (256, 128, 12320)])
-@pytest.mark.parametrize("spread", ["even", "some", "fifth", "half", "late", "first", "zeros", "rows"])
+@pytest.mark.parametrize("spread", ["even", "some", "fifth", "half", "late", "first", "zeros", "rows", "weights", "tiny_rows",
+                                    "tiny_columns", "zero_rows"])
 def test_products_of_halves_and_what_they_do_not_hold(gpu, M, N, K, spread):
     """Split products keep the componentwise error of test_products_off_the_sixteen_byte_grid whatever the magnitudes: values
     that half-precision parts of a tile's scale do not hold in no slice of k, in some, in every fifth (more than a workgroup
     notes at 12320 k), in half of them, behind a first slice of another magnitude or of zeros; zeros among the values; rows of
-    very different magnitude in a tile.  Two products in one call (no k ranges), each with every layout of its operands.  Where
-    some terms are 2^60 and more times the others, a sum is hardly more than its largest term, rounded with every product that
+    very different magnitude in a tile; one operand with values far below its largest (the weights of a peaked softmax, with
+    zeros behind the diagonal) against ordinary ones, and with rows or columns altogether that small.  Two products in one call (no k ranges), each with every layout of its operands.  Where
+    some terms are many times the others (2^60 and more, or a peak of the weights), a sum is hardly more than its largest term, rounded with every product that
     follows: there the bound is that of test_matmul_random_shapes_through_the_dispatch."""
     import torch
     gen = torch.Generator(device="cuda")
@@ -1001,7 +1003,17 @@ def test_products_of_halves_and_what_they_do_not_hold(gpu, M, N, K, spread):
 
     a_kr = torch.stack([spread_out(torch.randn((K, M), generator=gen, device="cuda")) for _ in range(2)])
     b_kc = torch.stack([spread_out(torch.randn((K, N), generator=gen, device="cuda") * 0.02) for _ in range(2)])
-    bound = 2e-6 if spread in ("some", "fifth", "half") else 4 * 1.2e-7
+    if spread == "weights":
+        seen = torch.arange(K, device="cuda")[:, None] <= torch.arange(M, device="cuda") * K // M
+        a_kr = torch.softmax((8.0 * a_kr).masked_fill(~seen, float("-inf")), dim=1)
+    elif spread == "tiny_rows":
+        a_kr[:, :, ::5] *= 2.0 ** -40
+    elif spread == "tiny_columns":
+        b_kc[:, :, 3::7] *= 2.0 ** -50
+    elif spread == "zero_rows":
+        a_kr[:, 10:20, ::3] *= 2.0 ** -30
+        a_kr[:, :, 5::9] = 0.0
+    bound = 2e-6 if spread in ("some", "fifth", "half", "weights") else 4 * 1.2e-7
     want = a_kr.double().transpose(1, 2) @ b_kc.double()
     scale = a_kr.double().abs().transpose(1, 2) @ b_kc.double().abs()
     for a in (a_kr.transpose(1, 2), a_kr.transpose(1, 2).contiguous()):

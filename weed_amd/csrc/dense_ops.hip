@@ -466,18 +466,30 @@ template <int OP> __device__ __forceinline__ float wave_reduce(float v)
     return v;
 }
 
+// The memory-side cache holds 256 MB of what was read or written last.  Passes over something larger that all run from its
+// beginning never meet any of it; a pass that begins where the one before it ended reads up to half of a 512 MB tensor
+// from the cache (a copy in place over 512 MB: 193 us a pass in one direction, 146 in turns; 1 GB 395 and 348; up to 256 MB, all
+// of it cached, 62.3 and 62.9).  A kernel does not know who ran before it, so the directions are fixed by what follows what
+// in a dense attention: the scores' product upwards, their scaling (multiplication or division) downwards, the mask's
+// addition upwards, the softmax downwards, the weights' product upwards.
+constexpr uint64_t kMemorySideCache = 256ull << 20;
+
 // Short contiguous rows (a causal prefill's scores: [B * heads * T] rows of at most a few thousand key positions):
 // one WAVEFRONT per row, four rows per workgroup, so no lane idles on a 64..2048-element row and nothing goes
 // through LDS.  V = 4: float4 accesses (every row 16-byte aligned, length a multiple of 4), V = 1: scalar.  The first
 // CACHED * 64 * V elements of a row stay in registers between the two passes.
-template <int V, int CACHED, bool FITS>
+// PASSING: more than the memory-side cache holds, from the last row to the first (see kMemorySideCache), and read past the
+// cache where it is written elsewhere, so that what stays there is the weights that the next product begins with.
+template <int V, int CACHED, bool FITS, bool PASSING = false>
 __global__ void __launch_bounds__(256) softmax_wave_rows_kernel(const float *__restrict__ a, float *__restrict__ out,
                                                                 AxisGeom g)
 {
     const uint32_t lane = threadIdx.x & 63U;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t nvec = g.axis_len / V;
-    for (uint32_t row = blockIdx.x * 4U + wave; row < g.rows; row += gridDim.x * 4U) {
+    const bool once = PASSING && a != out;
+    for (uint32_t done = blockIdx.x * 4U + wave; done < g.rows; done += gridDim.x * 4U) {
+        const uint32_t row = PASSING ? g.rows - 1U - done : done;
         uint64_t a_base, o_base;
         row_bases(g, row, a_base, o_base);
         const float *ap = a + a_base;
@@ -488,8 +500,12 @@ __global__ void __launch_bounds__(256) softmax_wave_rows_kernel(const float *__r
         for (int c = 0; c < CACHED; ++c) {
             const uint32_t idx = lane + 64U * c;
             if (V == 4) {
-                const float4 v = idx < nvec ? reinterpret_cast<const float4 *>(ap)[idx]
-                                            : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+                typedef float f4 __attribute__((ext_vector_type(4)));
+                f4 v = { -INFINITY, -INFINITY, -INFINITY, -INFINITY };
+                if (idx < nvec) {
+                    const f4 *p = reinterpret_cast<const f4 *>(ap) + idx;
+                    v = once ? __builtin_nontemporal_load(p) : *p;
+                }
                 cache[c][0] = v.x;
                 cache[c][V > 1 ? 1 : 0] = v.y;
                 cache[c][V > 2 ? 2 : 0] = v.z;
@@ -954,6 +970,7 @@ struct RowGeom {
     FastDiv dim[kRowDims - 1]; // the outer dimensions
     uint32_t row;   // elements of the contiguous dimension
     uint32_t n;     // pieces in all
+    uint32_t backwards; // from the last 1024 pieces to the first: see kMemorySideCache
     uint32_t a_stride[kRowDims - 1], b_stride[kRowDims - 1], o_stride[kRowDims - 1];
 };
 
@@ -969,7 +986,9 @@ __global__ void __launch_bounds__(256) elementwise_rows_kernel(const float *__re
                                                                float *out, RowGeom g)
 {
     constexpr bool kBinary = OP >= 1 && OP <= 5;
-    for (uint64_t base = (uint64_t)blockIdx.x * 1024U; base < g.n; base += (uint64_t)gridDim.x * 1024U) {
+    const uint64_t last = (g.n - 1U) / 1024U * 1024U;
+    for (uint64_t done = (uint64_t)blockIdx.x * 1024U; done < g.n; done += (uint64_t)gridDim.x * 1024U) {
+        const uint64_t base = g.backwards ? last - done : done;
         float x[4][4], y[4][4];
         uint64_t at[4];
         uint32_t count[4];
@@ -1399,6 +1418,7 @@ int weed_hip_elementwise_f32(int op, uint32_t rank, const uint32_t *shape, const
             n *= r.dim[dd - 1].d;
         }
         r.n = (uint32_t)n;
+        r.backwards = (op == WEED_HIP_EW_MUL || op == WEED_HIP_EW_DIV) && 4ull * g.n > kMemorySideCache;
         const uint32_t rb = (uint32_t)std::min<uint64_t>((n + 1023) / 1024, 256u * 16u);
         const float *ap = a_dev + a_off, *bp = unary ? ap : b + b_off;
         float *op_out = out_dev + o_off;
@@ -1520,7 +1540,11 @@ int weed_hip_softmax_f32(uint32_t rank, const uint32_t *shape, uint32_t axis, co
         }
     } else if (how == AXIS_WAVE_VEC) {
         // (kWaveRowMax = 8 * 4 * 64: such a row always fits a wavefront's registers)
-        softmax_wave_rows_kernel<4, 8, true><<<wave_row_blocks(g.rows), 256, 0, stream()>>>(a_dev, out_dev, g);
+        if (4ull * g.rows * g.axis_len > kMemorySideCache) {
+            softmax_wave_rows_kernel<4, 8, true, true><<<wave_row_blocks(g.rows), 256, 0, stream()>>>(a_dev, out_dev, g);
+        } else {
+            softmax_wave_rows_kernel<4, 8, true><<<wave_row_blocks(g.rows), 256, 0, stream()>>>(a_dev, out_dev, g);
+        }
     } else if (how == AXIS_WAVE && g.axis_len <= 128U) {
         if (g.axis_len <= 8U) {
             WEED_SHORT_ROWS(1, 2, 4);
@@ -1531,7 +1555,13 @@ int weed_hip_softmax_f32(uint32_t rank, const uint32_t *shape, uint32_t axis, co
         }
 #undef WEED_SHORT_ROWS
     } else if (how == AXIS_WAVE) {
-        if (g.axis_len <= 16U * 64U) {
+        if (4ull * g.rows * g.axis_len > kMemorySideCache) {
+            if (g.axis_len <= 16U * 64U) {
+                softmax_wave_rows_kernel<1, 16, true, true><<<wave_row_blocks(g.rows), 256, 0, stream()>>>(a_dev, out_dev, g);
+            } else {
+                softmax_wave_rows_kernel<1, 16, false, true><<<wave_row_blocks(g.rows), 256, 0, stream()>>>(a_dev, out_dev, g);
+            }
+        } else if (g.axis_len <= 16U * 64U) {
             softmax_wave_rows_kernel<1, 16, true><<<wave_row_blocks(g.rows), 256, 0, stream()>>>(a_dev, out_dev, g);
         } else {
             softmax_wave_rows_kernel<1, 16, false><<<wave_row_blocks(g.rows), 256, 0, stream()>>>(a_dev, out_dev, g);
