@@ -999,6 +999,64 @@ def test_chunks_of_many_rows(gpu, d, Hkv, Hq, mapping):
     cache.close()
 
 
+@pytest.mark.parametrize("lloyd,d,Hq,T,k_bits,v_bits,sign,mapping", [
+    (True, 64, 32, 64, 3, 4, 0, "blocked"),    # 256 rows of a KV head, all of a workgroup's
+    (True, 64, 64, 31, 2, 3, 1, "weed"),       # 248: the last tile is half full
+    (True, 80, 64, 25, 4, 4, 1, "blocked"),    # 200, thirteen tiles, the fewest; fields of five bits
+    (True, 100, 128, 29, 3, 4, 0, "weed"),     # 464, two groups of rows, the second one shorter
+    (True, 128, 32, 64, 3, 4, 0, "blocked"),
+    (False, 128, 64, 30, 8, 8, 0, "blocked"),  # 240
+    (False, 96, 32, 59, 6, 6, 0, "weed"),      # 236
+    (False, 64, 64, 32, 7, 7, 0, "blocked"),
+])
+def test_chunks_that_share_the_unpacking(gpu, lloyd, d, Hq, T, k_bits, v_bits, sign, mapping):
+    """A hundred rows and more per KV head over blocks enough for every workgroup to keep its tables and queries for a
+    while: positions of a chunk as calls of one position give them, also over fewer tokens than are cached, and the first
+    position of a sequence as long as the chunk.  Lloyd-Max tables: 4e-6 per side, as in test_chunks_of_many_rows.  Uniform
+    cells: a sum of codes cancels against the lower end of their range, 1.6 beside results of about 1/80, and fp32 sums of up to
+    28000 terms stray by some 4 * 2^-24 of their size: 4 * 2^-24 * 1.6 * 80 per side."""
+    import torch
+    S, Hkv = 7, 8
+    lens = [T, 65, 64, 1000, 4000, 23456, 28000]
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(d + Hq + T)
+    cache = gpu.KVCache(gpu.KV_LLOYDMAX if lloyd else gpu.KV_UNIFORM, S, Hkv, d, max(lens), k_bits, v_bits, sign, sign)
+    if not lloyd:
+        cache.set_scales(1.6, 1.6)
+    rk, rv = (torch.zeros(d * d, device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    gpu.make_rotation(5, d, rk)
+    gpu.make_rotation(6, d, rv)
+    cache.set_rotations(rk, rv)
+    for s, n in enumerate(lens):
+        k, v = (torch.randn((1, Hkv, n, d), generator=gen, device="cuda") for _ in range(2))
+        torch.cuda.synchronize()
+        cache.encode_append(k, v, seq_begin=s, rotate=1)
+        gpu.sync()
+    q = torch.randn((S, T, Hq, d), generator=gen, device="cuda")
+    gqa = gpu.GQA_WEED if mapping == "weed" else gpu.GQA_BLOCKED
+    flags = gpu.ATTN_ROTATE_Q | gpu.ATTN_UNROTATE_OUT
+    bar = 8e-6 if lloyd else 2 * 4 * 2.0 ** -24 * 1.6 * 80
+    for seen in (lens, [T, T, 64, 70, 3999, 640, 27000]):
+        seen = [max(n, T) for n in seen]
+        seen_dev = torch.tensor(seen, dtype=torch.int32, device="cuda")
+        out = torch.full_like(q, float("nan"))
+        torch.cuda.synchronize()
+        cache.decode_attn_chunk(q, out, lens=seen_dev if seen != lens else None, gqa_mapping=gqa, flags=flags)
+        gpu.sync()
+        assert not torch.isnan(out).any()
+        for t in sorted({0, 1, T // 2, T - 1}):
+            until = seen_dev - (T - 1 - t)
+            one, want = q[:, t].contiguous(), torch.zeros((S, Hq, d), device="cuda")
+            torch.cuda.synchronize()
+            cache.decode_attn_prefix(until, one, want, gqa_mapping=gqa, flags=flags)
+            gpu.sync()
+            for s in range(S):
+                rel = float((out[s, t] - want[s]).double().norm() / want[s].double().norm())
+                assert rel <= bar, "sequence %d of %d tokens, position %d: %.2e" % (s, seen[s], t, rel)
+    cache.close()
+
+
 @pytest.mark.parametrize("d,T", [(64, 28), (64, 40), (128, 28), (128, 40), (192, 28), (192, 40), (256, 28), (256, 40)])
 def test_merges_of_many_rows_by_rows_and_by_tiles(gpu, d, T):
     """9 x 28 x 16 rows rotate by tiles and merge by rows, 9 x 40 x 16 rows do both by tiles, several partials a row:

@@ -1328,6 +1328,19 @@ uint32_t pass_workgroups(uint32_t passes, uint32_t blocks, uint32_t waves)
     return best;
 }
 
+// Where the workgroups share the unpacking of the cache: thirteen tiles of rows and more per group of sixteen, so that seven of a
+// workgroup's eight wavefronts have rows (132 rows of 128 63 us by passes, 89 so), and as many blocks as it takes to earn what a
+// workgroup's start (tables, LDS, one round of workgroups that waits for the slowest) and a region's start in it (queries, partials, the
+// first block's way) cost more than by passes.  Measured at 52 to 64 positions x 32 heads on 8 (by passes -> shared, us):
+//   head_dim 128, K 3 + V 4 bits: 16 sequences of 2100 tokens 120 -> 131, 4096 205 -> 180; 40 of 2500 354 -> 314; 64 of 2176 495 -> 426;
+//     10 of 5200 159 -> 162; 8 of 100 to 10000 144 -> 157, of 100 to 16000 213 -> 202; 40 of 100 to 2500 239 -> 312
+//   head_dim 64: 16 of 2100 76 -> 78, of 6000 165 -> 140; 96: 100 -> 103 and 217 -> 186; 32: of 6000 114 -> 117 (left to the passes)
+//   fields beyond four bits at 128, dearer to unpack: 8 of 3000, K and V 5 bits 143 -> 114, 8 bits 125 -> 100, V alone 5 bits 115 -> 106;
+//     64 of 1500 571 -> 379, 529 -> 341 and 424 -> 341; 40 of 100 to 2500, V alone 278 -> 293; at 64, 8 bits, 8 of 3000 56 -> 62
+constexpr uint32_t kTilesToShare = 13;
+struct ShareCost { uint32_t workgroup, region; }; // in blocks
+constexpr ShareCost kNarrowFields{ 20, 24 }, kWideFields{ 8, 15 };
+
 // `lens_dev` (optional): attend over these per-sequence lengths instead of the cached ones.
 // `n_tokens` > 1: a chunk of query positions per sequence, the last `n_tokens` of the attended tokens being the
 // chunk's own (position t sees all but the last n_tokens - 1 - t); q_tstride / o_tstride step between positions.
@@ -1367,6 +1380,19 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
     // ONE copy of the process-wide tuning for the whole plan: weed_hip_kv_decode_tuning may change it from another host
     // thread at any time, and a plan must not pair a block count chosen under one setting with a search mode of another.
     const DecodeTuning tune = decode_tuning();
+    // Rows of a KV head that would take many passes share the unpacking of the cache instead (kv_decode_chunk.hip): groups of up to
+    // 256 rows, one run of blocks per workgroup and one round of workgroups.  (See kTilesToShare.)
+    const uint32_t row_tiles = (G + 15) / 16, most_tiles = mfma_decode_shared_rows / 16;
+    const uint32_t row_groups = (row_tiles + most_tiles - 1) / most_tiles, group_wgs = std::max(1u, 256u / row_groups);
+    bool shared = use_mfma && d >= 64 && d <= 128 && row_tiles >= kTilesToShare * row_groups && tune.wavefronts == 0;
+    if (shared) {
+        uint64_t blocks = 0;
+        for (int32_t l : c->lens) {
+            blocks += ((uint64_t)l + 63) / 64 * Hkv;
+        }
+        const ShareCost cost = d == 128 && (c->k.w > 4 || c->v.w > 4) ? kWideFields : kNarrowFields;
+        shared = blocks >= (uint64_t)group_wgs * cost.workgroup + (uint64_t)S * Hkv * cost.region;
+    }
     uint32_t n_splits, split_tokens = 0;
     uint32_t total_blocks = 0;
     RunGeom runs = { 1, 0, 8, 0 };
@@ -1523,7 +1549,11 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
         const uint32_t skew_pct = tune.skew_percent >= 0 ? (uint32_t)std::min(90, tune.skew_percent)
                                                          : (runs.waves == 12 ? kRunSkewPercent3 : kRunSkewPercent);
         const uint32_t nblk = virtual_blocks ? virtual_blocks : (max_len + 63) / 64;
-        for (;;) {
+        if (shared) {
+            // (a region of no more partials than the kernel behind merges by tiles)
+            runs = RunGeom{ std::max((total_blocks + group_wgs - 1) / group_wgs, (nblk + 62) / 63), 0, 8, 0 };
+        }
+        for (; !shared;) {
             runs.skew = std::min(runs.unit_blocks - 1, (runs.unit_blocks * skew_pct + 50) / 100);
             const uint32_t shortest = runs.unit_blocks - runs.skew;
             n_splits = (nblk + shortest - 1) / shortest + 1; // partial slots per (sequence, head)
@@ -1532,6 +1562,9 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
             }
             // one very long region and few of them: longer runs (fewer wavefronts) keep the merge within its limit
             runs.unit_blocks += std::max(1u, runs.unit_blocks / 8);
+        }
+        if (shared) {
+            n_splits = (nblk + runs.unit_blocks - 1) / runs.unit_blocks + 1;
         }
     } else {
         // split the context so that the launch has a few workgroups per compute unit
@@ -1762,7 +1795,14 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
         mp.tile_rows = pass_heads;
         ProfileScope prof("kv_decode_attn", timed);
         mp.grid_passes = 0;
-        if (passes > 1 && total_blocks && !fused_merge && !fused_query) {
+        if (shared) {
+            mp.head_first = 0;
+            mp.tile_rows = mp.G = (row_tiles + row_groups - 1) / row_groups * 16;
+            mp.grid_passes = row_groups;
+            if (total_blocks) {
+                WEED_HIP_TRY(launch_mfma_decode_shared(mp, d, stream()));
+            }
+        } else if (passes > 1 && total_blocks && !fused_merge && !fused_query) {
             // every pass in ONE launch: the passes' workgroups that read the same blocks run next to each other on one
             // XCD, so the cache is fetched from memory once instead of once per pass
             mp.grid_passes = passes;

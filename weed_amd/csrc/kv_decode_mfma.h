@@ -285,5 +285,10 @@ constexpr uint32_t mfma_decode_waves_per_wg(uint32_t gp, uint32_t d, uint32_t wk
 // Wavefronts per workgroup of the kernel instance that serves this shape (one workgroup fills a compute unit).
 uint32_t mfma_decode_workgroup_waves(uint32_t G, uint32_t d, uint32_t wk, uint32_t wv);
 int launch_mfma_decode(const MfmaParams &p, uint32_t d, hipStream_t s);
+// Many rows per KV head at head_dims 64, 96 and 128 (kv_decode_chunk.hip): `tile_rows` (at most mfma_decode_shared_rows) of them per
+// workgroup, `grid_passes` groups of rows, one run of `runs.unit_blocks` blocks per workgroup (no skew, nothing merged or rotated
+// there).
+constexpr uint32_t mfma_decode_shared_rows = 256;
+int launch_mfma_decode_shared(const MfmaParams &p, uint32_t d, hipStream_t s);
 
 } // namespace weedhip
