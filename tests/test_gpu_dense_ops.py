@@ -517,6 +517,67 @@ def test_elementwise_rows_of_pieces(gpu, shape, a_shape, b_shape):
     np.testing.assert_array_equal(acc.cpu().numpy(), np.broadcast_to(a + b, shape))
 
 
+@pytest.mark.parametrize("shape,b_shape,strided", [
+    ((8, 1025, 1025), (1025, 1025), False),           # two whole groups of repeats, rows of no whole pieces
+    ((11, 1030, 1028), (1030, 1028), True),           # three left over; rows 1029 apart: three dimensions
+    ((9, 2, 1100, 515), (2, 1100, 515), True),        # one left over; four dimensions
+    ((17, 2001, 2000), (2001, 2000), False),          # above the memory-side cache, no groups; divisions downwards
+    ((17, 2001, 2000), (1,), False),
+])
+def test_elementwise_masks_over_many_heads(gpu, shape, b_shape, strided):
+    """An operand of more than 4 MB repeated along the outermost dimension, and results beyond 256 MB: single IEEE operations,
+    exact against the CPU, in place and into another tensor, nothing written beside it."""
+    import torch
+    gen = torch.Generator().manual_seed(sum(shape))
+    a = torch.randn(shape, generator=gen)
+    b = torch.rand(b_shape, generator=gen) + 0.5
+    bd = b.cuda()
+
+    def room(value):
+        if not strided:
+            flat = torch.full((a.numel() + 8,), value, device="cuda")
+            return flat, flat[4:-4].view(shape)
+        wide = torch.full(shape[:-1] + (shape[-1] + 1,), value, device="cuda")
+        return wide, wide[..., :-1]
+
+    for op, want in ((gpu.EW_ADD, a + b), (gpu.EW_SUB, a - b), (gpu.EW_MUL, a * b), (gpu.EW_DIV, a / b)):
+        ad, (buf, out) = a.cuda(), room(-7.0)
+        torch.cuda.synchronize()
+        gpu.elementwise(op, ad, bd, out)
+        gpu.elementwise(op, ad, bd, ad)
+        gpu.sync()
+        assert torch.equal(out.cpu(), want) and torch.equal(ad.cpu(), want), op
+        assert int((buf != -7.0).sum()) <= a.numel()
+        if strided:
+            assert bool((buf[..., -1] == -7.0).all())
+        else:
+            assert bool((buf[:4] == -7.0).all()) and bool((buf[-4:] == -7.0).all())
+
+
+@pytest.mark.parametrize("rows,n", [(33001, 2048), (33001, 2047), (70001, 1001)])
+def test_softmax_of_more_than_the_memory_side_cache(gpu, rows, n):
+    """Short rows beyond 256 MB (whole 16-byte pieces, single elements, rows that a wavefront's registers do not hold), into another
+    tensor and in place, a row of the lowest values and one with infinities below.  Against float64: an exponential of a
+    difference of up to 12 errs by 12 * 2^-24 and 2 ulp, the sum and the quotient by less than 6 ulp."""
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(rows + n)
+    x = torch.randn((rows, n), generator=gen, device="cuda")
+    x[5] = torch.finfo(torch.float32).min
+    x[rows - 1, 3:] = -float("inf")
+    out = torch.full_like(x, -7.0)
+    torch.cuda.synchronize()
+    gpu.softmax(x, out, 1)
+    gpu.sync()
+    for first in range(0, rows, 10000):
+        part = x[first:first + 10000].double()
+        want = torch.softmax(part, 1)
+        err = ((out[first:first + 10000].double() - want).abs() - 20 * 2.0 ** -24 * want).max().item()
+        assert err <= 2.0 ** -126, (first, err)
+    gpu.softmax(x, x, 1)
+    gpu.sync()
+    assert torch.equal(x, out)
+
+
 def test_elementwise_broadcast_and_gather(gpu):
     """add / sub / mul / div are single IEEE operations, so they must equal numpy bit for bit, including with a
     broadcast (stride 0) operand, transposed views and an output that aliases the first operand."""

@@ -974,6 +974,37 @@ struct RowGeom {
     uint32_t a_stride[kRowDims - 1], b_stride[kRowDims - 1], o_stride[kRowDims - 1];
 };
 
+// `count` (1 to 4) elements of a row that is contiguous, or one value for all of them.
+__device__ __forceinline__ void fetch_piece(const float *p, bool row, uint32_t count, float (&v)[4])
+{
+    if (row && count == 4U) {
+        const ew_f4u q = *reinterpret_cast<const ew_f4u *>(p);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = q[e];
+        }
+    } else {
+        const float first = p[0];
+#pragma unroll
+        for (uint32_t e = 0; e < 4; ++e) {
+            v[e] = row && e && e < count ? p[e] : first;
+        }
+    }
+}
+__device__ __forceinline__ void store_piece(float *p, uint32_t count, ew_f4u v)
+{
+    if (count == 4U) {
+        *reinterpret_cast<ew_f4u *>(p) = v;
+    } else {
+#pragma unroll
+        for (uint32_t e = 0; e < 3; ++e) {
+            if (e < count) {
+                p[e] = v[e];
+            }
+        }
+    }
+}
+
 // Broadcasts and views whose innermost dimension is contiguous in the output and contiguous or repeated in the operands
 // (the prefill's scores / sqrt(d) and scores + mask, a bias row): a thread takes 16-byte pieces of a row, four at a time
 // and 4 KB apart, so that a workgroup walks 16 KB in one stretch as elementwise_flat_kernel does.  HBM-bound, 8 bytes
@@ -1012,24 +1043,9 @@ __global__ void __launch_bounds__(256) elementwise_rows_kernel(const float *__re
                 oi += (uint64_t)k * g.o_stride[dd];
             }
             at[u] = oi;
-            auto fetch = [&](const float *p, bool row, float (&v)[4]) {
-                if (row && count[u] == 4U) {
-                    const ew_f4u q = *reinterpret_cast<const ew_f4u *>(p);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        v[e] = q[e];
-                    }
-                } else {
-                    const float first = p[0];
-#pragma unroll
-                    for (uint32_t e = 0; e < 4; ++e) {
-                        v[e] = row && e && e < count[u] ? p[e] : first;
-                    }
-                }
-            };
-            fetch(a + ai, A_ROW, x[u]);
+            fetch_piece(a + ai, A_ROW, count[u], x[u]);
             if (kBinary) {
-                fetch(b + bi, B_ROW, y[u]);
+                fetch_piece(b + bi, B_ROW, count[u], y[u]);
             }
         }
 #pragma unroll
@@ -1039,15 +1055,60 @@ __global__ void __launch_bounds__(256) elementwise_rows_kernel(const float *__re
             for (int e = 0; e < 4; ++e) {
                 v[e] = elementwise_apply<OP>(x[u][e], kBinary ? y[u][e] : x[u][e]);
             }
-            if (count[u] == 4U) {
-                *reinterpret_cast<ew_f4u *>(out + at[u]) = v;
-            } else {
+            store_piece(out + at[u], count[u], v);
+        }
+    }
+}
+
+// The same where the second operand repeats along the outermost dimension (a mask over heads; `repeats` of it, the last of the
+// geometry's dimensions counting groups of kRepeats): a thread takes one piece of kRepeats of them and reads the second
+// operand's piece once.  Inside the memory-side cache the operand's reads weigh as much as the result's: a mask over 16 heads
+// of 2000 x 2000 109 -> 86 us, 32 of 1500 119 -> 101, 16 of 1030 30.4 -> 24.6, 8 of 1100 16.7 -> 15.2.  Not for operands that an
+// XCD's L2 holds (32 heads of 1024 x 1024 40.4 -> 43.5, of 700 23.1 -> 23.7), for fewer than two groups (4 heads of 1536 13.3 -> 14.6), nor
+// beyond the memory-side cache, where kRepeats streams cost more than the reads (32 heads of 2048 208 -> 232; of 2000, in a
+// prefill, no gain).  Eight repeats at once: 84, 98 and 24 us for the first three, 242 for the last; fewer heads qualify.
+constexpr uint32_t kRepeats = 4U;
+constexpr uint64_t kRepeatedBytes = 4ull << 20;
+template <int OP>
+__global__ void __launch_bounds__(256) elementwise_repeat_kernel(const float *__restrict__ a, const float *__restrict__ b,
+                                                                 float *out, RowGeom g, uint32_t repeats, uint32_t a_rep,
+                                                                 uint32_t o_rep)
+{
+    const uint64_t last = (g.n - 1U) / 256U * 256U;
+    for (uint64_t done = (uint64_t)blockIdx.x * 256U; done < g.n; done += (uint64_t)gridDim.x * 256U) {
+        const uint64_t piece = (g.backwards ? last - done : done) + threadIdx.x;
+        if (piece >= g.n) {
+            continue;
+        }
+        uint32_t rest = g.pieces.div((uint32_t)piece), first = 0;
+        const uint32_t c = ((uint32_t)piece - rest * g.pieces.d) * 4U, count = min(4U, g.row - c);
+        uint64_t ai = c, bi = c, oi = c;
 #pragma unroll
-                for (uint32_t e = 0; e < 3; ++e) {
-                    if (e < count[u]) {
-                        out[at[u] + e] = v[e];
-                    }
+        for (int dd = 0; dd < kRowDims - 1; ++dd) {
+            const uint32_t q = g.dim[dd].div(rest), k = rest - q * g.dim[dd].d;
+            rest = q;
+            ai += (uint64_t)k * g.a_stride[dd];
+            bi += (uint64_t)k * g.b_stride[dd];
+            oi += (uint64_t)k * g.o_stride[dd];
+            first = k * kRepeats; // (the last dimension's stays)
+        }
+        float y[4], x[kRepeats][4];
+#pragma unroll
+        for (uint32_t u = 0; u < kRepeats; ++u) {
+            if (first + u < repeats) {
+                fetch_piece(a + ai + (uint64_t)(first + u) * a_rep, true, count, x[u]);
+            }
+        }
+        fetch_piece(b + bi, true, count, y);
+#pragma unroll
+        for (uint32_t u = 0; u < kRepeats; ++u) {
+            if (first + u < repeats) {
+                ew_f4u v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    v[e] = elementwise_apply<OP>(x[u][e], y[e]);
                 }
+                store_piece(out + oi + (uint64_t)(first + u) * o_rep, count, v);
             }
         }
     }
@@ -1422,6 +1483,25 @@ int weed_hip_elementwise_f32(int op, uint32_t rank, const uint32_t *shape, const
         const uint32_t rb = (uint32_t)std::min<uint64_t>((n + 1023) / 1024, 256u * 16u);
         const float *ap = a_dev + a_off, *bp = unary ? ap : b + b_off;
         float *op_out = out_dev + o_off;
+        const uint32_t top = g.rank - 1U; // the outermost dimension
+        if (!unary && top && g.a_stride[0] && g.b_stride[0] && g.b_stride[top] == 0U && g.shape[top] >= 2U * kRepeats &&
+            4ull * (g.n / g.shape[top]) > kRepeatedBytes && 4ull * g.n <= kMemorySideCache) {
+            const uint32_t groups = (g.shape[top] + kRepeats - 1U) / kRepeats;
+            // (the dimension to the last place; the ones between are of length 1)
+            r.dim[top - 1U] = FastDiv::of(1U);
+            r.dim[kRowDims - 2] = FastDiv::of(groups);
+            r.a_stride[kRowDims - 2] = r.b_stride[kRowDims - 2] = r.o_stride[kRowDims - 2] = 0U; // (a_rep, o_rep)
+            r.n = (uint32_t)(n / g.shape[top] * groups);
+            const uint32_t wgs = (uint32_t)std::min<uint64_t>((r.n + 255ull) / 256ull, 256u * 16u);
+            with_elementwise_op(op, [&](auto kOp) {
+                if constexpr (kOp.value >= 1 && kOp.value <= 5) {
+                    elementwise_repeat_kernel<kOp.value><<<wgs, 256, 0, stream()>>>(ap, bp, op_out, r, g.shape[top],
+                                                                                    g.a_stride[top], g.o_stride[top]);
+                }
+            });
+            WEED_HIP_LAUNCH_CHECK();
+            return WEED_HIP_OK;
+        }
         with_elementwise_op(op, [&](auto kOp) {
             constexpr int OP = kOp.value;
             if (g.a_stride[0] && (unary || g.b_stride[0])) {
