@@ -466,15 +466,15 @@ def extras(capi, torch, workloads, steps, warmup):
     C = torch.empty((4096, 4096), device="cuda").t()
     secs, kernel_s, how = time_one_kernel_op(capi, torch, lambda: capi.matmul(A, W, C), "matmul", steps, warmup)
     flops = 2.0 * 4096 * 1024 * 4096
-    # The product runs on the 16-bit matrix instruction with both operands split into two half-precision parts and three
-    # products of parts per fp32 product, so its matrix-core bound is that instruction's peak over three; the same product on
+    # The product runs on the bfloat16 matrix instruction with both operands split exactly into three parts and six
+    # products of parts per fp32 product, so its matrix-core bound is the bfloat16 peak over six; the same product on
     # the fp32 instruction (weed_hip_matmul_tuning) is measured beside it against that instruction's own peak.
-    split_peak = 2500.0 / 3.0
+    split_peak = 2500.0 / 6.0
     out["cfg5b_matmul_f32_4096x1024x4096"] = {
         "tflops": flops / secs / 1e12, "kernel_ms": 1e3 * kernel_s, "kernel_tflops": flops / kernel_s / 1e12,
         "roofline": {"bound": "mfma", "achieved": flops / kernel_s / 1e12, "peak": split_peak, "unit": "TFLOP/s",
                      "frac": flops / kernel_s / 1e12 / split_peak,
-                     "peak_is": "16-bit dense 2500 TFLOP/s / 3 products of half-precision parts per fp32 product",
+                     "peak_is": "bf16 dense 2500 TFLOP/s / 6 products of bfloat16 parts per fp32 product",
                      "frac_of_fp32_instruction_peak_157.3": flops / kernel_s / 1e12 / 157.3}}
     out["cfg5b_matmul_f32_4096x1024x4096"].update(how)
     capi.matmul_tuning(True)

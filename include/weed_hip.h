@@ -92,25 +92,21 @@ int weed_hip_matmul_f32(uint32_t M, uint32_t N, uint32_t K, const float *a_dev, 
 /* Which matrix instruction the large products run on (no counterpart in the reference; process-wide, takes effect
  * with the next call).  0, the default: products of at least 17 rows and columns whose operands are contiguous along
  * one dimension (of 17 to 64 rows against a k-contiguous weight with 256 k or more: those of 512 columns or more, and
- * off the 16-byte grid those of a k too long for the streaming kernel) run on the 16-bit matrix instructions with both
- * operands split: as three products of half-precision parts (of 11 bits each, behind a power-of-two scale per tile of
- * the operand) where a slice of 32 k holds no values above 2^6 of the largest in the tile's first 64 k and values below
- * 2^-22 of it in one operand at most, and otherwise, as the products of 17 to 64 rows throughout, as six of the nine
- * products of three exact bfloat16 parts; accumulated in fp32 either way.  Twice the fp32 instruction's speed and more.  The error against the exact product is
- * no larger than the fp32 instruction's own: 2.2e-7 of the result's norm for normal operands at k = 4096, 1.2e-7 at k =
- * 768 (5.0e-7 and 1.3e-7 as six products); relative to sum_k |a_ik| |b_kj| per element, for operands spanning
- * 2^-20 .. 2^20 at k = 1028, where the slices go by six products, largest 7.1e-7 against 5.9e-7 and mean 5.8e-8
- * against 5.1e-8.  Two things the split does not keep: an operand that is not finite gives NaN where the fp32
- * instruction would give an infinity, and operand values below 2^-112 in magnitude lose accuracy where they go by
- * bfloat16 parts, because their second and third parts fall below bfloat16's normal range and the
+ * off the 16-byte grid those of a k too long for the streaming kernel) run on the bfloat16 instruction with both
+ * operands split exactly into three bfloat16 parts and six of the nine products of parts accumulated in fp32 -- 1.5
+ * times the fp32 instruction's speed and more.  The error against the exact product is the fp32 instruction's own:
+ * relative to sum_k |a_ik| |b_kj| per element, at k = 1028 over operands spanning 2^-20 .. 2^20, largest 7.1e-7
+ * against 5.9e-7 and mean 5.8e-8 against 5.1e-8; for operands of one magnitude 8.0e-8 against 1.0e-7 and 9.1e-9
+ * against 1.1e-8 (a sequential fp32 sum: 3.4e-7 and 2.0e-8).  Two things the split does not keep: an operand that is
+ * not finite gives NaN where the fp32 instruction would give an infinity, and operand values below 2^-112 in
+ * magnitude lose accuracy, because their second and third parts fall below bfloat16's normal range and the
  * instruction takes them as zeros (largest error 1.3e-6 for values around 2^-115, 3e-5 around 2^-120, 9e-4 around
  * 2^-125; fp32 denormals count as zero), where the fp32 instruction keeps 2e-7 down to the denormals.  Where every
  * operand is 16-byte aligned in all its rows or columns that is the default's result; products off that grid (sizes,
  * strides or addresses that are no multiples of four elements) look at what they multiply and take the sums of such a
  * tile of the output again on the fp32 instruction, so that they keep infinities and tiny values whichever is chosen.
  * 1: the fp32 instruction everywhere (v_mfma_f32_32x32x2_f32: every product exact, sums rounded to fp32 in ascending
- * k per 16-k slice).  Products with at most 16 rows, operands strided in both dimensions and strides of 2^22 elements and
- * more do not depend on it.
+ * k per 16-k slice).  Products with at most 16 rows, and operands strided in both dimensions, do not depend on it.
  * The process-wide default is read once from the environment variable WEED_HIP_MATMUL_FP32 (1 = the fp32
  * instruction). */
 int weed_hip_matmul_tuning(int32_t fp32_instruction);

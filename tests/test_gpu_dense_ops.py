@@ -1036,13 +1036,15 @@ def test_whole_tiles_in_k_ranges_with_half_a_slice(gpu, M, N, K):
 @pytest.mark.parametrize("spread", ["even", "some", "fifth", "half", "late", "first", "zeros", "rows", "weights", "tiny_rows",
                                     "tiny_columns", "zero_rows"])
 def test_products_of_halves_and_what_they_do_not_hold(gpu, M, N, K, spread):
-    """Split products keep the componentwise error of test_products_off_the_sixteen_byte_grid whatever the magnitudes: values
-    that half-precision parts of a tile's scale do not hold in no slice of k, in some, in every fifth (more than a workgroup
-    notes at 12320 k), in half of them, behind a first slice of another magnitude or of zeros; zeros among the values; rows of
-    very different magnitude in a tile; one operand with values far below its largest (the weights of a peaked softmax, with
-    zeros behind the diagonal) against ordinary ones, and with rows or columns altogether that small.  Two products in one call (no k ranges), each with every layout of its operands.  Where
-    some terms are many times the others (2^60 and more, or a peak of the weights), a sum is hardly more than its largest term, rounded with every product that
-    follows: there the bound is that of test_matmul_random_shapes_through_the_dispatch."""
+    """Split products keep the componentwise error of test_products_off_the_sixteen_byte_grid whatever the magnitudes, those that
+    two half-precision parts of a value would not hold among them: in no slice of k, in some, in every fifth, in half of them, behind a
+    first slice of another magnitude or of zeros; zeros among the values; rows of very different magnitude in a tile; one operand
+    with values far below its largest (the weights of a peaked softmax, with zeros behind the diagonal) against ordinary ones, and
+    with rows or columns altogether that small.  Two products in one call (no k ranges), each with every layout of its operands.
+    Where some terms are many times the others (2^60 and more, or a peak of the weights), a sum is hardly more than its largest
+    term, rounded with every product that follows: there the bound is that of test_matmul_random_shapes_through_the_dispatch,
+    2e-6 for up to 4096 k.  Six roundings per 16 k at random directions, each of 2^-24 / sqrt(3) of the sum at most, are 1.3e-6 as
+    a standard deviation there and 2.3e-6 at 12320 k, so behind 4096 k the bound of the weights grows with the root of k."""
     import torch
     gen = torch.Generator(device="cuda")
     gen.manual_seed(M + N + K)
@@ -1075,6 +1077,8 @@ def test_products_of_halves_and_what_they_do_not_hold(gpu, M, N, K, spread):
         a_kr[:, 10:20, ::3] *= 2.0 ** -30
         a_kr[:, :, 5::9] = 0.0
     bound = 2e-6 if spread in ("some", "fifth", "half", "weights") else 4 * 1.2e-7
+    if spread == "weights":
+        bound *= max(1.0, K / 4096.0) ** 0.5
     want = a_kr.double().transpose(1, 2) @ b_kc.double()
     scale = a_kr.double().abs().transpose(1, 2) @ b_kc.double().abs()
     for a in (a_kr.transpose(1, 2), a_kr.transpose(1, 2).contiguous()):
@@ -1089,7 +1093,7 @@ def test_products_of_halves_and_what_they_do_not_hold(gpu, M, N, K, spread):
 
 @pytest.mark.parametrize("along_rows", [True, False])
 def test_products_with_long_strides(gpu, along_rows):
-    """Strides beyond the reach of the split-operand tiles' 32-bit offsets go by the fp32 instruction."""
+    """Rows or columns 16 MB and more apart, of which a tile's last lie beyond what a 32-bit offset in bytes reaches."""
     import torch
     M, N, K, stride = 20, 24, 40, (1 << 22) + 8
     gen = torch.Generator(device="cuda")
@@ -1105,3 +1109,96 @@ def test_products_with_long_strides(gpu, along_rows):
     gpu.sync()
     scale = a.double().abs() @ b.double().abs()
     assert float(((out.double() - a.double() @ b.double()).abs() / scale).max()) <= 4 * 1.2e-7
+
+
+@pytest.mark.parametrize("M,N,K", [(128, 128, 256), (256, 384, 1024), (130, 133, 260), (71, 515, 2051)])
+@pytest.mark.parametrize("mirrored", [False, True])
+def test_split_products_with_one_term_a_sum(gpu, M, N, K, mirrored):
+    """Sums of a single term, whole tiles, k ranges and sizes off the 16-byte grid: a column taken by a one is the column bit for
+    bit, whatever the magnitudes beside it (2^-90 to 1: three exact parts lie in bfloat16's normal range); integers of 12 bits
+    are multiplied exactly; and a product of two values errs by the products of parts that are left out, 2^-23 of it, and two
+    roundings."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+    rows, cols = (N, M) if mirrored else (M, N)
+    take = torch.randint(0, K, (cols,), generator=gen, device="cuda")
+    j = torch.arange(cols, device="cuda")
+    dense = torch.randn((rows, K), generator=gen, device="cuda")
+    wide = dense * torch.exp2(torch.randint(-90, 1, (rows, K), generator=gen, device="cuda").float())
+    whole = torch.randint(2048, 4096, (rows, K), generator=gen, device="cuda").float()
+    factor = torch.randn((cols,), generator=gen, device="cuda")
+    for name, full, value in (("ones", dense, torch.ones_like(factor)), ("ones", wide, torch.ones_like(factor)),
+                              ("integers", whole, torch.full_like(factor, 2049.0)), ("factors", dense, factor)):
+        sparse = torch.zeros((K, cols), device="cuda")
+        sparse[take, j] = value
+        want = full[:, take].double() * value.double()
+        left, right = (sparse.t(), full.t()) if mirrored else (full, sparse)
+        for a in (left.contiguous(), left.t().contiguous().t()):
+            for b in (right.contiguous(), right.t().contiguous().t()):
+                out = torch.zeros((N, M), device="cuda").t()
+                torch.cuda.synchronize()
+                gpu.matmul(a, b, out)
+                gpu.sync()
+                got = (out.t() if mirrored else out).double()
+                if name == "factors":
+                    assert bool(((got - want).abs() <= 2.0 ** -22 * want.abs()).all()), (a.stride(), b.stride())
+                else:
+                    assert torch.equal(got, want), (name, a.stride(), b.stride())
+
+
+@pytest.mark.parametrize("M,N,K", [(128, 128, 256), (132, 260, 2084), (130, 133, 260), (71, 515, 2051)])
+@pytest.mark.parametrize("mirrored", [False, True])
+@pytest.mark.parametrize("spread", ["blocks_30", "blocks_45", "blocks_90", "scattered"])
+def test_split_products_of_values_that_meet_zeros(gpu, M, N, K, mirrored, spread):
+    """Small values of one operand that meet the other one's values where the large ones meet zeros: a grouped weight against
+    features of two magnitudes, and a sparse one against magnitudes from 2^-60 to 1.  The componentwise bound of
+    test_products_off_the_sixteen_byte_grid for the first; where terms of a sum differ by so much (see
+    test_products_of_halves_and_what_they_do_not_hold) that of test_matmul_random_shapes_through_the_dispatch."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+    rows, cols = (N, M) if mirrored else (M, N)
+    full, other = torch.randn((rows, K), generator=gen, device="cuda"), torch.randn((K, cols), generator=gen, device="cuda")
+    if spread == "scattered":
+        full *= torch.exp2(torch.randint(-60, 1, (rows, K), generator=gen, device="cuda").float())
+        other[torch.rand(other.shape, generator=gen, device="cuda") < 0.98] = 0.0
+    else:
+        full[:, K // 4:] *= 2.0 ** -int(spread[7:])
+        other[:K // 4, cols // 2:] = 0.0
+        other[K // 4:, :cols // 2] = 0.0
+    left, right = (other.t(), full.t()) if mirrored else (full, other)
+    want, scale = left.double() @ right.double(), left.double().abs() @ right.double().abs()
+    bound = 2e-6 if spread == "scattered" else 4 * 1.2e-7
+    for a in (left.contiguous(), left.t().contiguous().t()):
+        for b in (right.contiguous(), right.t().contiguous().t()):
+            out = torch.zeros((N, M), device="cuda").t()
+            torch.cuda.synchronize()
+            gpu.matmul(a, b, out)
+            gpu.sync()
+            err = float(((out.double() - want).abs() / scale.clamp_min(1e-300)).max())
+            assert bool(out.isfinite().all()) and err <= bound, (a.stride(), b.stride(), err)
+
+
+@pytest.mark.parametrize("M,N,K", [(130, 133, 260), (71, 515, 2051)])
+@pytest.mark.parametrize("mirrored", [False, True])
+def test_products_off_the_sixteen_byte_grid_of_tiny_values_that_meet_zeros(gpu, M, N, K, mirrored):
+    """Off the 16-byte grid values around 2^-110 beside ordinary ones keep the accuracy of the fp32 instruction where only they
+    meet anything but zeros."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+    rows, cols = (N, M) if mirrored else (M, N)
+    full, other = torch.randn((rows, K), generator=gen, device="cuda"), torch.randn((K, cols), generator=gen, device="cuda")
+    full[:, K // 4:] *= 2.0 ** -110
+    other[:K // 4, cols // 2:] = 0.0
+    left, right = (other.t(), full.t()) if mirrored else (full, other)
+    want, scale = left.double() @ right.double(), left.double().abs() @ right.double().abs()
+    for a in (left.contiguous(), left.t().contiguous().t()):
+        for b in (right.contiguous(), right.t().contiguous().t()):
+            out = torch.zeros((N, M), device="cuda").t()
+            torch.cuda.synchronize()
+            gpu.matmul(a, b, out)
+            gpu.sync()
+            err = float(((out.double() - want).abs() / scale).max())
+            assert err <= 4 * 1.2e-7, (a.stride(), b.stride(), err)

@@ -290,7 +290,7 @@ def matmul(a, b, out):
 
 
 def matmul_tuning(fp32_instruction=False):
-    """Large products on the fp32 matrix instruction (True) or as 16-bit products of split operands (default)."""
+    """Large products on the fp32 matrix instruction (True) or as six bfloat16 products of split operands (default)."""
     check(load().weed_hip_matmul_tuning(1 if fp32_instruction else 0))
 
 
