@@ -1057,6 +1057,49 @@ def test_chunks_that_share_the_unpacking(gpu, lloyd, d, Hq, T, k_bits, v_bits, s
     cache.close()
 
 
+_PLANS = """
+import json, sys
+import torch
+from weed_amd import capi
+capi.check(capi.load().weed_hip_init(0))
+for lloyd, d, Hq, T, k_bits, v_bits, sign, mapping, lens in json.loads(sys.argv[1]):
+    cache = capi.KVCache(capi.KV_LLOYDMAX if lloyd else capi.KV_UNIFORM, len(lens), 8, d, max(lens), k_bits, v_bits, sign, sign)
+    if not lloyd:
+        cache.set_scales(1.6, 1.6)
+    for s, n in enumerate(lens):
+        k = torch.randn((1, 8, n, d), device="cuda")
+        torch.cuda.synchronize()
+        cache.encode_append(k, k, seq_begin=s, rotate=0)
+        capi.sync()
+    q = torch.randn((len(lens), T, Hq, d), device="cuda")
+    out = torch.zeros_like(q)
+    torch.cuda.synchronize()
+    cache.decode_attn_chunk(q, out, gqa_mapping=capi.GQA_WEED if mapping == "weed" else capi.GQA_BLOCKED, flags=0)
+    capi.sync()
+    cache.close()
+"""
+
+
+def test_plans_of_chunks_that_share_the_unpacking(gpu):
+    """Every case of the test above is served by the workgroups that it is about, in groups of up to 256 rows as even as tiles of
+    sixteen allow, and one of them with fewer blocks is not; as the plan says that a process with WEED_HIP_DECODE_PLAN=1 prints."""
+    import json
+    import os
+    import re
+    import subprocess
+    import sys
+    cases = [m for m in test_chunks_that_share_the_unpacking.pytestmark if m.name == "parametrize"][0].args[1]
+    calls = [list(c) + [[c[3], 65, 64, 1000, 4000, 23456, 28000]] for c in cases] + [list(cases[0]) + [[500] * 7]]
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    done = subprocess.run([sys.executable, "-c", _PLANS, json.dumps(calls)], cwd=root, capture_output=True, text=True, timeout=100,
+                          env=dict(os.environ, WEED_HIP_DECODE_PLAN="1"))
+    assert done.returncode == 0, done.stderr[-2000:]
+    plans = [(int(a), int(b)) for a, b in re.findall(r"groups that share the unpacking (\d+) of (\d+) rows", done.stderr)]
+    rows = [c[2] * c[3] // 8 for c in cases]
+    groups = [-(-r // 256) for r in rows]
+    assert plans == [(g, -(-(-(-r // 16)) // g) * 16) for r, g in zip(rows, groups)] + [(0, 0)]
+
+
 @pytest.mark.parametrize("d,T", [(64, 28), (64, 40), (128, 28), (128, 40), (192, 28), (192, 40), (256, 28), (256, 40)])
 def test_merges_of_many_rows_by_rows_and_by_tiles(gpu, d, T):
     """9 x 28 x 16 rows rotate by tiles and merge by rows, 9 x 40 x 16 rows do both by tiles, several partials a row:

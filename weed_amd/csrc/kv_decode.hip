@@ -1384,6 +1384,7 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
     // 256 rows, one run of blocks per workgroup and one round of workgroups.  (See kTilesToShare.)
     const uint32_t row_tiles = (G + 15) / 16, most_tiles = mfma_decode_shared_rows / 16;
     const uint32_t row_groups = (row_tiles + most_tiles - 1) / most_tiles, group_wgs = std::max(1u, 256u / row_groups);
+    const uint32_t group_rows = (row_tiles + row_groups - 1) / row_groups * 16;
     bool shared = use_mfma && d >= 64 && d <= 128 && row_tiles >= kTilesToShare * row_groups && tune.wavefronts == 0;
     if (shared) {
         uint64_t blocks = 0;
@@ -1731,9 +1732,10 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
         std::fprintf(stderr,
                      "%s: S %u Hkv %u G %u d %u bits %u/%u  matrix cores %d  passes %u  blocks %u  run %u (skew %u, in turns %u) "
                      "x %u wavefronts  whole regions per workgroup %u  workgroups per region %u  general merge %d  "
-                     "queries in the kernel %d  slots %u\n",
+                     "queries in the kernel %d  slots %u  groups that share the unpacking %u of %u rows\n",
                      fn, S, Hkv, G, d, c->k.w, c->v.w, (int)use_mfma, passes, total_blocks, runs.unit_blocks, runs.skew,
-                     runs.group_cycles, runs.waves, wg_regions, region_wgs, (int)general_merge, (int)fused_query, n_splits);
+                     runs.group_cycles, runs.waves, wg_regions, region_wgs, (int)general_merge, (int)fused_query, n_splits,
+                     shared ? row_groups : 0U, shared ? group_rows : 0U);
     }
     // (the kernels that take one (sequence, head) row per workgroup have the sequence on a 16-bit grid dimension)
     // (prep_q_kernel puts one more row on that dimension when it also builds the block offsets)
@@ -1797,7 +1799,7 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
         mp.grid_passes = 0;
         if (shared) {
             mp.head_first = 0;
-            mp.tile_rows = mp.G = (row_tiles + row_groups - 1) / row_groups * 16;
+            mp.tile_rows = mp.G = group_rows;
             mp.grid_passes = row_groups;
             if (total_blocks) {
                 WEED_HIP_TRY(launch_mfma_decode_shared(mp, d, stream()));
