@@ -105,6 +105,67 @@ def test_noalloc_refuses_shapes_beyond_its_workspace(gpu):
     cache.close()
 
 
+def _long_cache(gpu, S, Hkv, tokens, room):
+    """A cache of S sequences with room for `room` tokens, and what appends `tokens` normal ones to each."""
+    import torch
+    cache = gpu.KVCache(gpu.KV_LLOYDMAX, S, Hkv, 128, room, 3, 4)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(S + tokens)
+
+    def append(n):
+        k, v = (torch.randn((S, Hkv, n, 128), generator=gen, device="cuda") for _ in range(2))
+        torch.cuda.synchronize()
+        cache.encode_append(k, v, rotate=0)
+        gpu.sync()
+
+    append(tokens)
+    return cache, append
+
+
+def test_noalloc_takes_what_the_passes_leave_room_for(gpu):
+    """256 heads on one KV head over blocks enough to share their unpacking, which needs a workspace of 40 MB where the passes
+    take 28: within the static workspace, so both entry points take the call, with the same bits."""
+    import torch
+    cache, _ = _long_cache(gpu, 16, 1, 22100, 22100)
+    q = torch.randn((16, 256, 128), device="cuda")
+    ref, out = torch.zeros_like(q), torch.full_like(q, float("nan"))
+    torch.cuda.synchronize()
+    cache.decode_attn(q, ref, gqa_mapping=gpu.GQA_BLOCKED, flags=0)
+    cache.decode_attn_noalloc(q, out, gqa_mapping=gpu.GQA_BLOCKED, flags=0)
+    gpu.sync()
+    assert bool(torch.isfinite(ref).all()) and torch.equal(ref, out)
+    cache.close()
+
+
+def test_a_captured_chunk_keeps_to_the_workspace_it_finds(gpu):
+    """A chunk whose cache has grown, since its workspace was allocated, past where chunks share the unpacking, which takes more
+    of it: captured and replayed in what is there; eager calls afterwards let it grow, and agree."""
+    import torch
+    S, Hkv, T, Hq = 2, 8, 64, 32
+    cache, append = _long_cache(gpu, S, Hkv, 21000, 22100)
+    q = torch.randn((S, T, Hq, 128), device="cuda")
+    warm, out, eager = torch.zeros_like(q), torch.full_like(q, float("nan")), torch.zeros_like(q)
+    torch.cuda.synchronize()
+    cache.decode_attn_chunk(q, warm, gqa_mapping=gpu.GQA_BLOCKED, flags=0)
+    append(1100)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.current_stream()):
+        cache.decode_attn_chunk(q, out, gqa_mapping=gpu.GQA_BLOCKED, flags=0)
+    first = None
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        gpu.sync()
+        first = out.clone() if first is None else first
+        assert torch.equal(out, first)
+    del graph
+    cache.decode_attn_chunk(q, eager, gqa_mapping=gpu.GQA_BLOCKED, flags=0)
+    gpu.sync()
+    # (8e-6: the bound of test_chunks_that_share_the_unpacking)
+    assert float((first - eager).double().norm() / eager.double().norm()) <= 8e-6
+    cache.close()
+
+
 @pytest.mark.parametrize("n_seq,ctx", [(1, 2048), (8, 1024), (3, 1000)])
 def test_noalloc_call_replayed_from_a_graph(gpu, oracle, n_seq, ctx):
     """The allocation-free entry point under graph capture: the captured call is one kernel whose workgroups count

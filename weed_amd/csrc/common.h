@@ -18,6 +18,8 @@ int fail(int code, const char *fmt, ...);
 
 // The stream every launch goes to.
 hipStream_t stream();
+// Whether that stream is being captured into a graph: a call then neither allocates nor waits.
+bool capturing();
 
 // Ensures weed_hip_init() ran (device 0 by default).  Returns a WEED_HIP_* status.
 int ensure_init();

@@ -104,6 +104,12 @@ int fail(int code, const char *fmt, ...)
 
 hipStream_t stream() { return g_stream; }
 
+bool capturing()
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(stream(), &status) == hipSuccess && status != hipStreamCaptureStatusNone;
+}
+
 int current_device() { return g_initialised ? g_device : -1; }
 
 int ensure_init()

@@ -1394,6 +1394,19 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
         const ShareCost cost = d == 128 && (c->k.w > 4 || c->v.w > 4) ? kWideFields : kNarrowFields;
         shared = blocks >= (uint64_t)group_wgs * cost.workgroup + (uint64_t)S * Hkv * cost.region;
     }
+    // workspace: rotated q (fp32), its fp16 hi / lo halves, per-head scale and sum, split partials
+    const size_t n_q = (size_t)S * Hq * d;
+    const size_t q_bytes = sizeof(float) * n_q;
+    const size_t h_bytes = (sizeof(uint16_t) * n_q + 15) / 16 * 16;
+    const size_t s_bytes = (sizeof(float) * (size_t)S * Hq + 15) / 16 * 16;
+    const size_t off_bytes = (sizeof(uint32_t) * ((size_t)S + 1) + 15) / 16 * 16;
+    // (the arrival counters of the kernel's own merge come first, at the same place whatever the shape, because they
+    // have to be zero when a launch starts: they are cleared when the workspace is allocated and every launch leaves
+    // them at zero; the static scratch starts as zeros)
+    const size_t arrive_bytes = sizeof(uint32_t) * kMfmaMergeCounters;
+    const auto workspace = [&](uint32_t slots) {
+        return arrive_bytes + q_bytes + 2 * h_bytes + 2 * s_bytes + off_bytes + sizeof(float) * (size_t)S * Hq * slots * (d + 2);
+    };
     uint32_t n_splits, split_tokens = 0;
     uint32_t total_blocks = 0;
     RunGeom runs = { 1, 0, 8, 0 };
@@ -1550,11 +1563,7 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
         const uint32_t skew_pct = tune.skew_percent >= 0 ? (uint32_t)std::min(90, tune.skew_percent)
                                                          : (runs.waves == 12 ? kRunSkewPercent3 : kRunSkewPercent);
         const uint32_t nblk = virtual_blocks ? virtual_blocks : (max_len + 63) / 64;
-        if (shared) {
-            // (a region of no more partials than the kernel behind merges by tiles)
-            runs = RunGeom{ std::max((total_blocks + group_wgs - 1) / group_wgs, (nblk + 62) / 63), 0, 8, 0 };
-        }
-        for (; !shared;) {
+        for (;;) {
             runs.skew = std::min(runs.unit_blocks - 1, (runs.unit_blocks * skew_pct + 50) / 100);
             const uint32_t shortest = runs.unit_blocks - runs.skew;
             n_splits = (nblk + shortest - 1) / shortest + 1; // partial slots per (sequence, head)
@@ -1565,7 +1574,19 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
             runs.unit_blocks += std::max(1u, runs.unit_blocks / 8);
         }
         if (shared) {
-            n_splits = (nblk + runs.unit_blocks - 1) / runs.unit_blocks + 1;
+            // (a region of no more partials than the kernel behind merges by tiles)
+            const RunGeom own = { std::max((total_blocks + group_wgs - 1) / group_wgs, (nblk + 62) / 63), 0, 8, 0 };
+            const uint32_t own_splits = (nblk + own.unit_blocks - 1) / own.unit_blocks + 1;
+            // These runs are up to twice as many as the passes' (256 workgroups' against 16 of eight wavefronts), and so are the
+            // partials.  A call whose workspace holds the passes' only goes by passes: under capture, where it cannot grow, and a
+            // call of one position up to the static scratch, which its twin that allocates nothing has, with the same bits.
+            const auto only_passes_fit = [&](size_t room) { return workspace(own_splits) > room && workspace(n_splits) <= room; };
+            shared = !(n_tokens == 1 && only_passes_fit(kStaticScratchBytes)) &&
+                     !(!fixed_ws && only_passes_fit(c->dec_ws_bytes) && capturing());
+            if (shared) {
+                runs = own;
+                n_splits = own_splits;
+            }
         }
     } else {
         // split the context so that the launch has a few workgroups per compute unit
@@ -1578,18 +1599,7 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
     }
     WEED_HIP_REQUIRE(n_splits <= kMaxSlots, "%s: internal split count %u too large", fn, n_splits);
 
-    // workspace: rotated q (fp32), its fp16 hi / lo halves, per-head scale and sum, split partials
-    const size_t n_q = (size_t)S * Hq * d;
-    const size_t q_bytes = sizeof(float) * n_q;
-    const size_t h_bytes = (sizeof(uint16_t) * n_q + 15) / 16 * 16;
-    const size_t s_bytes = (sizeof(float) * (size_t)S * Hq + 15) / 16 * 16;
-    const size_t part_bytes = sizeof(float) * (size_t)S * Hq * n_splits * (d + 2);
-    const size_t off_bytes = (sizeof(uint32_t) * ((size_t)S + 1) + 15) / 16 * 16;
-    // (the arrival counters of the kernel's own merge come first, at the same place whatever the shape, because they
-    // have to be zero when a launch starts: they are cleared when the workspace is allocated and every launch leaves
-    // them at zero; the static scratch starts as zeros)
-    const size_t arrive_bytes = sizeof(uint32_t) * kMfmaMergeCounters;
-    const size_t need = arrive_bytes + q_bytes + 2 * h_bytes + 2 * s_bytes + off_bytes + part_bytes;
+    const size_t need = workspace(n_splits);
     if (fixed_ws) {
         // the caller's workspace (the static scratch): nothing is allocated, larger shapes are refused
         WEED_HIP_REQUIRE(need <= fixed_ws_bytes,
