@@ -1090,6 +1090,8 @@ def test_plans_of_chunks_that_share_the_unpacking(gpu):
     import sys
     cases = [m for m in test_chunks_that_share_the_unpacking.pytestmark if m.name == "parametrize"][0].args[1]
     calls = [list(c) + [[c[3], 65, 64, 1000, 4000, 23456, 28000]] for c in cases] + [list(cases[0]) + [[500] * 7]]
+    # three, five, six and seven groups: the runs of all of them in one round of workgroups of the compute units of an XCD
+    calls += [[True, 64, hq, t, 3, 4, 0, "blocked", [12000] * 4] for hq, t in ((104, 50), (168, 60), (208, 59), (216, 64))]
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     done = subprocess.run([sys.executable, "-c", _PLANS, json.dumps(calls)], cwd=root, capture_output=True, text=True, timeout=100,
                           env=dict(os.environ, WEED_HIP_DECODE_PLAN="1"))
@@ -1097,7 +1099,12 @@ def test_plans_of_chunks_that_share_the_unpacking(gpu):
     plans = [(int(a), int(b)) for a, b in re.findall(r"groups that share the unpacking (\d+) of (\d+) rows", done.stderr)]
     rows = [c[2] * c[3] // 8 for c in cases]
     groups = [-(-r // 256) for r in rows]
-    assert plans == [(g, -(-(-(-r // 16)) // g) * 16) for r, g in zip(rows, groups)] + [(0, 0)]
+    assert plans[:-4] == [(g, -(-(-(-r // 16)) // g) * 16) for r, g in zip(rows, groups)] + [(0, 0)]
+    assert [g for g, _ in plans[-4:]] == [3, 5, 6, 7]
+    runs = re.findall(r"  blocks (\d+)  run (\d+) ", done.stderr)
+    assert len(runs) == len(plans)
+    for (blocks, run), (g, _) in zip(runs, plans):
+        assert g == 0 or -(-(-(-int(blocks) // int(run))) // 8) * g <= 32, (blocks, run, g)
 
 
 @pytest.mark.parametrize("d,T", [(64, 28), (64, 40), (128, 28), (128, 40), (192, 28), (192, 40), (256, 28), (256, 40)])

@@ -1383,8 +1383,11 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
     // Rows of a KV head that would take many passes share the unpacking of the cache instead (kv_decode_chunk.hip): groups of up to
     // 256 rows, one run of blocks per workgroup and one round of workgroups.  (See kTilesToShare.)
     const uint32_t row_tiles = (G + 15) / 16, most_tiles = mfma_decode_shared_rows / 16;
-    const uint32_t row_groups = (row_tiles + most_tiles - 1) / most_tiles, group_wgs = std::max(1u, 256u / row_groups);
-    const uint32_t group_rows = (row_tiles + row_groups - 1) / row_groups * 16;
+    const uint32_t row_groups = (row_tiles + most_tiles - 1) / most_tiles, group_rows = (row_tiles + row_groups - 1) / row_groups * 16;
+    // (one round on every XCD: the groups of a run lie on one, which has 32 compute units.  256 / groups in all instead put 33 to
+    // 36 workgroups on some of them with 3, 5, 6 or 7 groups, and those took two rounds: 648 rows of 96, 8 sequences of 5682
+    // tokens 246 us, 145 so, 156 by passes; 640 rows of 128, 2 of 70414 780, 440 and 499.)
+    const uint32_t group_wgs = 8 * std::max(1u, 32u / row_groups);
     bool shared = use_mfma && d >= 64 && d <= 128 && row_tiles >= kTilesToShare * row_groups && tune.wavefronts == 0;
     if (shared) {
         uint64_t blocks = 0;
