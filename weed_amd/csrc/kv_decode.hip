@@ -1331,15 +1331,34 @@ uint32_t pass_workgroups(uint32_t passes, uint32_t blocks, uint32_t waves)
 // Where the workgroups share the unpacking of the cache: thirteen tiles of rows and more per group of sixteen, so that seven of a
 // workgroup's eight wavefronts have rows (132 rows of 128 63 us by passes, 89 so), and as many blocks as it takes to earn what a
 // workgroup's start (tables, LDS, one round of workgroups that waits for the slowest) and a region's start in it (queries, partials, the
-// first block's way) cost more than by passes.  Measured at 52 to 64 positions x 32 heads on 8 (by passes -> shared, us):
-//   head_dim 128, K 3 + V 4 bits: 16 sequences of 2100 tokens 120 -> 131, 4096 205 -> 180; 40 of 2500 354 -> 314; 64 of 2176 495 -> 426;
-//     10 of 5200 159 -> 162; 8 of 100 to 10000 144 -> 157, of 100 to 16000 213 -> 202; 40 of 100 to 2500 239 -> 312
-//   head_dim 64: 16 of 2100 76 -> 78, of 6000 165 -> 140; 96: 100 -> 103 and 217 -> 186; 32: of 6000 114 -> 117 (left to the passes)
-//   fields beyond four bits at 128, dearer to unpack: 8 of 3000, K and V 5 bits 143 -> 114, 8 bits 125 -> 100, V alone 5 bits 115 -> 106;
-//     64 of 1500 571 -> 379, 529 -> 341 and 424 -> 341; 40 of 100 to 2500, V alone 278 -> 293; at 64, 8 bits, 8 of 3000 56 -> 62
+// first block's way) cost more than by passes.  A block takes a workgroup the same time for 13 tiles as for 16, and the passes 13
+// sixteenths: where the fields are cheap to unpack and a block's products long (96 and 128 coordinates) there is little to earn
+// with few tiles, and the line rises with the cube of that.  Fields beyond four bits are dearer by passes, bytes the least so.
+// Measured on 440 drawn calls around the lines, 17 to 64 positions, 200 to 2000 rows per KV head (by passes -> shared, us; below a
+// line by passes):
+//   head_dim 128, fields up to 4 bits: 13 tiles, 19 sequences of 5500-10600 tokens 199 -> 180; 14 tiles, 4 of 13451 142 -> 148
+//     (below); 16 tiles, 3 of 18000 164 -> 150, 16 of 4096 205 -> 180; 40 of 100-2500 239 -> 312 (below)
+//   96: 13 tiles, 8 of 17800-37500 125 -> 137 and 15 tiles, 2 of 22900 116 -> 124 (both below), 13 tiles, 4 of 52600 198 -> 207 (the
+//     furthest behind of those above); 16 tiles, 6 of 10300 148 -> 128
+//   64: 13 tiles, 41 of 200-6600 212 -> 200; 15, 58 of 3257 167 -> 144; 32: of 6000 114 -> 117 (left to the passes)
+//   5 to 7 bits at 64 and 96: 1.3 to 1.7 times as fast from the line on; bytes: 61 of 1900-3700 249 -> 255, 16 of 14657 124 -> 127
+//     (below), 18 of 13800 188 -> 174
+//   beyond 4 bits at 128: 8 of 3000, K and V 5 bits 143 -> 114, 8 bits 125 -> 100, V alone 5 bits 115 -> 106; 40 of 100 to 2500,
+//     V alone 278 -> 293
 constexpr uint32_t kTilesToShare = 13;
-struct ShareCost { uint32_t workgroup, region; }; // in blocks
-constexpr ShareCost kNarrowFields{ 20, 24 }, kWideFields{ 8, 15 };
+bool sharing_pays(uint32_t d, uint32_t widest_field, uint32_t tiles, uint32_t groups, uint32_t wgs, uint64_t regions, uint64_t blocks)
+{
+    double workgroup = 20.0, region = 24.0; // in blocks
+    if (widest_field > 4 && d == 128) {
+        workgroup = 8.0, region = 15.0;
+    } else if (widest_field == 8) {
+        workgroup = 32.0, region = 40.0;
+    } else if (widest_field <= 4 && d > 64) {
+        const double room = 16.0 * groups / tiles;
+        workgroup = (d == 96 ? 20.0 : 18.0) * room * room * room, region = 20.0;
+    }
+    return (double)blocks >= wgs * workgroup + (double)regions * region;
+}
 
 // `lens_dev` (optional): attend over these per-sequence lengths instead of the cached ones.
 // `n_tokens` > 1: a chunk of query positions per sequence, the last `n_tokens` of the attended tokens being the
@@ -1394,8 +1413,7 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
         for (int32_t l : c->lens) {
             blocks += ((uint64_t)l + 63) / 64 * Hkv;
         }
-        const ShareCost cost = d == 128 && (c->k.w > 4 || c->v.w > 4) ? kWideFields : kNarrowFields;
-        shared = blocks >= (uint64_t)group_wgs * cost.workgroup + (uint64_t)S * Hkv * cost.region;
+        shared = sharing_pays(d, std::max(c->k.w, c->v.w), row_tiles, row_groups, group_wgs, (uint64_t)S * Hkv, blocks);
     }
     // workspace: rotated q (fp32), its fp16 hi / lo halves, per-head scale and sum, split partials
     const size_t n_q = (size_t)S * Hq * d;
@@ -1586,6 +1604,9 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
             const auto only_passes_fit = [&](size_t room) { return workspace(own_splits) > room && workspace(n_splits) <= room; };
             shared = !(n_tokens == 1 && only_passes_fit(kStaticScratchBytes)) &&
                      !(!fixed_ws && only_passes_fit(c->dec_ws_bytes) && capturing());
+            // So do few regions of very many blocks, whose runs the limit on partials makes so long that workgroups are missing (one
+            // sequence of 230117 tokens, two KV heads of 96: 124 of them, 194 us against 129).
+            shared = shared && 8ull * own.unit_blocks <= 9ull * ((total_blocks + group_wgs - 1) / group_wgs);
             if (shared) {
                 runs = own;
                 n_splits = own_splits;
