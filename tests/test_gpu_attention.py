@@ -1082,8 +1082,8 @@ for lloyd, d, Hq, T, k_bits, v_bits, sign, mapping, Hkv, lens in json.loads(sys.
 
 def test_plans_of_chunks_that_share_the_unpacking(gpu):
     """Every case of the test above is served by the workgroups that it is about, in groups of up to 256 rows as even as tiles of
-    sixteen allow, and one of them with fewer blocks is not, nor are two whose rows or fields earn less and one of two regions
-    that would need more partials than are merged; as the plan says that a process with WEED_HIP_DECODE_PLAN=1 prints."""
+    sixteen allow, and one of them with fewer blocks is not, nor are two whose rows or fields earn less, one of two regions
+    that would need more partials than are merged and one of seventeen groups, half a round of workgroups; as the plan says that a process with WEED_HIP_DECODE_PLAN=1 prints."""
     import json
     import os
     import re
@@ -1092,7 +1092,7 @@ def test_plans_of_chunks_that_share_the_unpacking(gpu):
     cases = [m for m in test_chunks_that_share_the_unpacking.pytestmark if m.name == "parametrize"][0].args[1]
     calls = [list(c) + [8, [c[3], 65, 64, 1000, 4000, 23456, 28000]] for c in cases] + [list(cases[0]) + [8, [500] * 7]]
     calls += [[True, 96, 96, 17, 3, 4, 0, "blocked", 8, [15000] * 4], [False, 64, 32, 64, 8, 8, 0, "blocked", 8, [15000] * 4]]
-    calls += [[True, 64, 8, 64, 3, 4, 0, "blocked", 2, [170000]]]
+    calls += [[True, 64, 8, 64, 3, 4, 0, "blocked", 2, [170000]], [True, 64, 68, 64, 3, 4, 0, "blocked", 1, [40000]]]
     # three, five, six and seven groups: the runs of all of them in one round of workgroups of the compute units of an XCD
     calls += [[True, 64, hq, t, 3, 4, 0, "blocked", 8, [12000] * 4] for hq, t in ((104, 50), (168, 60), (208, 59), (216, 64))]
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -1102,7 +1102,7 @@ def test_plans_of_chunks_that_share_the_unpacking(gpu):
     plans = [(int(a), int(b)) for a, b in re.findall(r"groups that share the unpacking (\d+) of (\d+) rows", done.stderr)]
     rows = [c[2] * c[3] // 8 for c in cases]
     groups = [-(-r // 256) for r in rows]
-    assert plans[:-4] == [(g, -(-(-(-r // 16)) // g) * 16) for r, g in zip(rows, groups)] + 4 * [(0, 0)]
+    assert plans[:-4] == [(g, -(-(-(-r // 16)) // g) * 16) for r, g in zip(rows, groups)] + 5 * [(0, 0)]
     assert [g for g, _ in plans[-4:]] == [3, 5, 6, 7]
     runs = re.findall(r"  blocks (\d+)  run (\d+) ", done.stderr)
     assert len(runs) == len(plans)

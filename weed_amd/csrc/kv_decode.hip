@@ -1348,6 +1348,11 @@ uint32_t pass_workgroups(uint32_t passes, uint32_t blocks, uint32_t waves)
 constexpr uint32_t kTilesToShare = 13;
 bool sharing_pays(uint32_t d, uint32_t widest_field, uint32_t tiles, uint32_t groups, uint32_t wgs, uint64_t regions, uint64_t blocks)
 {
+    // (17 to 19 groups leave compute units idle, more than 32 take a second round: 4352 rows, 7 sequences of 7497 tokens, of 96
+    // 315 -> 344 us, of 64 254 -> 270; with 11 groups, 176 workgroups, it is 232 -> 208 still, at 8 bits with 17 554 -> 429)
+    if (widest_field <= 4 && (wgs * groups < 160 || wgs * groups > 256)) {
+        return false;
+    }
     double workgroup = 20.0, region = 24.0; // in blocks
     if (widest_field > 4 && d == 128) {
         workgroup = 8.0, region = 15.0;
