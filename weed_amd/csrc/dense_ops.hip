@@ -471,7 +471,9 @@ template <int OP> __device__ __forceinline__ float wave_reduce(float v)
 // from the cache (a copy in place over 512 MB: 193 us a pass in one direction, 146 in turns; 1 GB 395 and 348; up to 256 MB, all
 // of it cached, 62.3 and 62.9).  A kernel does not know who ran before it, so the directions are fixed by what follows what
 // in a dense attention: the scores' product upwards, their scaling (multiplication or division) downwards, the mask's
-// addition upwards, the softmax downwards, the weights' product upwards.
+// addition upwards, the softmax downwards, the weights' product upwards.  Any two passes in different directions gain (multiplication, tanh,
+// division of 288 MB 300 -> 279 us); one that is repeated alone meets nothing either way and loses up to 3 % downwards (a
+// multiplication from 288 MB into another 288 MB 102.5 -> 105.8, a division of 512 MB in place 189.5 -> 192.1).
 constexpr uint64_t kMemorySideCache = 256ull << 20;
 
 // Short contiguous rows (a causal prefill's scores: [B * heads * T] rows of at most a few thousand key positions):
@@ -1066,7 +1068,8 @@ __global__ void __launch_bounds__(256) elementwise_rows_kernel(const float *__re
 // of 2000 x 2000 109 -> 86 us, 32 of 1500 119 -> 101, 16 of 1030 30.4 -> 24.6, 8 of 1100 16.7 -> 15.2.  Not for operands that an
 // XCD's L2 holds (32 heads of 1024 x 1024 40.4 -> 43.5, of 700 23.1 -> 23.7), for fewer than two groups (4 heads of 1536 13.3 -> 14.6), nor
 // beyond the memory-side cache, where kRepeats streams cost more than the reads (32 heads of 2048 208 -> 232; of 2000, in a
-// prefill, no gain).  Eight repeats at once: 84, 98 and 24 us for the first three, 242 for the last; fewer heads qualify.
+// prefill, no gain).  Into another tensor 40 heads and more gain less (48 of 4.8 MB 101 -> 93 us) or lose (40 of 1100 x
+// 1100 72.5 -> 74.4; in place 65.4 -> 64.1).  Eight repeats at once: 84, 98 and 24 us for the first three, 242 for the last; fewer heads qualify.
 constexpr uint32_t kRepeats = 4U;
 constexpr uint64_t kRepeatedBytes = 4ull << 20;
 template <int OP>

@@ -1333,31 +1333,33 @@ uint32_t pass_workgroups(uint32_t passes, uint32_t blocks, uint32_t waves)
 // workgroup's start (tables, LDS, one round of workgroups that waits for the slowest) and a region's start in it (queries, partials, the
 // first block's way) cost more than by passes.  A block takes a workgroup the same time for 13 tiles as for 16, and the passes 13
 // sixteenths: where the fields are cheap to unpack and a block's products long (96 and 128 coordinates) there is little to earn
-// with few tiles, and the line rises with the cube of that.  Fields beyond four bits are dearer by passes, bytes the least so.
-// Measured on 440 drawn calls around the lines, 17 to 64 positions, 200 to 2000 rows per KV head (by passes -> shared, us; below a
+// with few tiles, and the line rises with the cube of that.  Fields beyond four bits are dearer by passes, but for bytes, which take no
+// table there, as uniform cells of up to four bits do: nothing to earn with either at 96, nor with bytes at 64.
+// Measured on 800 drawn calls around the lines, 17 to 64 positions, 200 to 2000 rows per KV head (by passes -> shared, us; below a
 // line by passes):
 //   head_dim 128, fields up to 4 bits: 13 tiles, 19 sequences of 5500-10600 tokens 199 -> 180; 14 tiles, 4 of 13451 142 -> 148
 //     (below); 16 tiles, 3 of 18000 164 -> 150, 16 of 4096 205 -> 180; 40 of 100-2500 239 -> 312 (below)
 //   96: 13 tiles, 8 of 17800-37500 125 -> 137 and 15 tiles, 2 of 22900 116 -> 124 (both below), 13 tiles, 4 of 52600 198 -> 207 (the
 //     furthest behind of those above); 16 tiles, 6 of 10300 148 -> 128
 //   64: 13 tiles, 41 of 200-6600 212 -> 200; 15, 58 of 3257 167 -> 144; 32: of 6000 114 -> 117 (left to the passes)
-//   5 to 7 bits at 64 and 96: 1.3 to 1.7 times as fast from the line on; bytes: 61 of 1900-3700 249 -> 255, 16 of 14657 124 -> 127
-//     (below), 18 of 13800 188 -> 174
+//   5 to 7 bits at 64 and 96: 1.3 to 1.7 times as fast from the line on; bytes at 96 (by passes): 16 of 14657 124 -> 127, 2 of
+//     39000-55000 182 -> 202, at 64 30 of 4700-9100 271 -> 283, 18 of 13800 188 -> 174; 4-bit cells at 96 (by passes): 4 of 36700-56000 180 -> 191
 //   beyond 4 bits at 128: 8 of 3000, K and V 5 bits 143 -> 114, 8 bits 125 -> 100, V alone 5 bits 115 -> 106; 40 of 100 to 2500,
 //     V alone 278 -> 293
 constexpr uint32_t kTilesToShare = 13;
-bool sharing_pays(uint32_t d, uint32_t widest_field, uint32_t tiles, uint32_t groups, uint32_t wgs, uint64_t regions, uint64_t blocks)
+bool sharing_pays(uint32_t d, bool cells, uint32_t widest_field, uint32_t tiles, uint32_t groups, uint32_t wgs, uint64_t regions, uint64_t blocks)
 {
     // (17 to 19 groups leave compute units idle, more than 32 take a second round: 4352 rows, 7 sequences of 7497 tokens, of 96
     // 315 -> 344 us, of 64 254 -> 270; with 11 groups, 176 workgroups, it is 232 -> 208 still, at 8 bits with 17 554 -> 429)
     if (widest_field <= 4 && (wgs * groups < 160 || wgs * groups > 256)) {
         return false;
     }
+    if ((widest_field == 8 && d < 128) || (cells && widest_field <= 4 && d == 96)) {
+        return false;
+    }
     double workgroup = 20.0, region = 24.0; // in blocks
     if (widest_field > 4 && d == 128) {
         workgroup = 8.0, region = 15.0;
-    } else if (widest_field == 8) {
-        workgroup = 32.0, region = 40.0;
     } else if (widest_field <= 4 && d > 64) {
         const double room = 16.0 * groups / tiles;
         workgroup = (d == 96 ? 20.0 : 18.0) * room * room * room, region = 20.0;
@@ -1418,7 +1420,8 @@ int decode_impl(const char *fn, weed_hip_kv_cache *c, int32_t n_q_heads, int32_t
         for (int32_t l : c->lens) {
             blocks += ((uint64_t)l + 63) / 64 * Hkv;
         }
-        shared = sharing_pays(d, std::max(c->k.w, c->v.w), row_tiles, row_groups, group_wgs, (uint64_t)S * Hkv, blocks);
+        shared = sharing_pays(d, c->cfg.mode == WEED_HIP_KV_UNIFORM, std::max(c->k.w, c->v.w), row_tiles, row_groups, group_wgs,
+                              (uint64_t)S * Hkv, blocks);
     }
     // workspace: rotated q (fp32), its fp16 hi / lo halves, per-head scale and sum, split partials
     const size_t n_q = (size_t)S * Hq * d;

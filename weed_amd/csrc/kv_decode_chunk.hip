@@ -6,7 +6,10 @@
 // head_dim 128, two blocks, one barrier per block), and every wavefront takes two tiles of sixteen rows against them, so that
 // an operand read from LDS serves both.  The matrix instructions (fp16 halves of queries and probabilities, as there) and the
 // softmax are what is left: 4096 and some 3500 cycles per SIMD for a block and 256 rows of 128, of 8900 that it takes -- matrix
-// and vector instructions of the two wavefronts of a SIMD overlap hardly at all.
+// and vector instructions of the two wavefronts of a SIMD overlap hardly at all, and at 128 with tables 180 bytes per lane of two tiles'
+// queries, sums, scores and probabilities go to scratch and back (256 registers are not enough; 20 bytes at 96 and with uniform cells).
+// The softmax, the split of the probabilities and the partials' write-out are those of kv_decode_mfma_kernel.h, for two tiles at a
+// time: a change to one is due in the other.
 // 64 positions x 32 heads on 8 of 128, K 3 + V 4 bits, 16 sequences: of 8192 tokens 360 -> 296 us, of 4096 205 -> 180, 4096 to 8192
 // 294 -> 257; 64 sequences of 1500, 5-bit fields 571 -> 379, 8-bit uniform ones 529 -> 341.  Where it is used: see kTilesToShare.
 // Against float64 its error is no larger (8192 tokens: Lloyd-Max 1.0e-6 against 1.1e-6, 8-bit cells 6e-6 against 10e-6).
