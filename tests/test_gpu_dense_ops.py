@@ -1203,3 +1203,21 @@ def test_products_off_the_sixteen_byte_grid_of_tiny_values_that_meet_zeros(gpu, 
             gpu.sync()
             err = float(((out.double() - want).abs() / scale).max())
             assert err <= 4 * 1.2e-7, (a.stride(), b.stride(), err)
+
+
+@pytest.mark.parametrize("batch,M,N,K", [(1, 1156, 132, 64), (1, 132, 1156, 40), (3, 1028, 260, 36), (1, 1285, 517, 33), (1, 264, 132, 2052),
+                                         (5, 129, 131, 95)])
+def test_split_products_tile_order(gpu, batch, M, N, K):
+    """More tiles of rows than a band holds, fewer tiles than XCDs, k ranges and products of a batch: every tile exactly once.
+
+    Products of integers up to 64 over these k are exact in every order, so nothing but a wrong tile can differ."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+    A = torch.randint(-64, 65, (1, batch, M, K), generator=gen, device="cuda").float()
+    B = torch.randint(-64, 65, (1, batch, N, K), generator=gen, device="cuda").float().transpose(2, 3)
+    C = torch.full((1, batch, M, N), 7.0, device="cuda")
+    gpu.matmul_batched(A, B, C) if batch > 1 else gpu.matmul(A[0, 0], B[0, 0], C[0, 0])
+    gpu.sync()
+    want = torch.stack([a.double().cpu() @ b.double().cpu() for a, b in zip(A[0], B[0])])
+    assert torch.equal(C[0].cpu().double(), want)
