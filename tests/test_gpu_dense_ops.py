@@ -1221,3 +1221,31 @@ def test_split_products_tile_order(gpu, batch, M, N, K):
     gpu.sync()
     want = torch.stack([a.double().cpu() @ b.double().cpu() for a, b in zip(A[0], B[0])])
     assert torch.equal(C[0].cpu().double(), want)
+
+
+@pytest.mark.parametrize("a_col,b_col,o_col", [(True, True, True), (True, False, False), (False, True, False), (False, False, True)])
+@pytest.mark.parametrize("M,N,K,infinite", [(4096, 4096, 544, False), (4092, 4088, 548, False), (4093, 4087, 547, False), (4093, 4087, 547, True),
+                                            (1804, 5124, 3996, False), (1803, 5123, 3997, False)])
+def test_split_products_in_large_tiles(gpu, a_col, b_col, o_col, M, N, K, infinite):
+    """Whole tiles of 256, checked loads, loads off the 16-byte grid, k ranges.
+
+    Sums of products of integers up to 32 over these k stay below 2^24: exact in every order.  An infinity in a row of a makes
+    that row what it is in float64 (infinities, NaN where it meets a zero) and no other one."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+
+    def matrix(rows, cols, col):
+        x = torch.randint(-32, 33, (cols, rows) if col else (rows, cols), generator=gen, device="cuda").float()
+        return x.t() if col else x
+
+    A, B = matrix(M, K, a_col), matrix(K, N, b_col)
+    if infinite:
+        A[M - 3, K - 1] = float("inf")
+    C = matrix(M, N, o_col)
+    bias = torch.randint(-32, 33, (N,), generator=gen, device="cuda").float()
+    torch.cuda.synchronize()
+    gpu.linear(A, B, bias, C)
+    gpu.sync()
+    want = A.double().contiguous() @ B.double().contiguous() + bias.double()
+    assert torch.equal(torch.nan_to_num(C.double(), nan=0.5), torch.nan_to_num(want, nan=0.5))
