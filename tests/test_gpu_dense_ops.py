@@ -1249,3 +1249,27 @@ def test_split_products_in_large_tiles(gpu, a_col, b_col, o_col, M, N, K, infini
     gpu.sync()
     want = A.double().contiguous() @ B.double().contiguous() + bias.double()
     assert torch.equal(torch.nan_to_num(C.double(), nan=0.5), torch.nan_to_num(want, nan=0.5))
+
+
+@pytest.mark.parametrize("fp32_instruction", [False, True])
+@pytest.mark.parametrize("M,N,K", [(128, 128, 2048), (200, 64, 736), (131, 66, 1027), (1000, 260, 4096)])
+def test_matmul_batched_of_one_product_over_k_ranges(gpu, M, N, K, fp32_instruction):
+    """One product of a longer batch: its k ranges are not the products behind it.  (The operands lie at the front of buffers
+    that hold more of them, so that a range taken for a product reads another one's values, not what lies beyond.)"""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+    more = 64
+    a = torch.randint(-16, 17, (1, more, M, K), generator=gen, device="cuda").float()[:, :1]
+    b = torch.randint(-16, 17, (1, more, N, K), generator=gen, device="cuda").float()[:, :1].transpose(2, 3)
+    out = torch.full((1, more, M, N), 7.0, device="cuda")
+    torch.cuda.synchronize()
+    gpu.load().weed_hip_matmul_tuning(int(fp32_instruction))
+    try:
+        gpu.matmul_batched(a, b, out[:, :1])
+        gpu.sync()
+    finally:
+        gpu.load().weed_hip_matmul_tuning(0)
+    # sums of integers below 2^24: exact in every order
+    assert torch.equal(out[0, 0].double().cpu(), a[0, 0].double().cpu() @ b[0, 0].double().cpu())
+    assert torch.all(out[:, 1:] == 7.0)
