@@ -1008,6 +1008,9 @@ def test_chunks_of_many_rows(gpu, d, Hkv, Hq, mapping):
     (False, 128, 64, 30, 8, 8, 0, "blocked"),  # 240
     (False, 96, 32, 59, 6, 6, 0, "weed"),      # 236
     (False, 64, 64, 32, 7, 7, 0, "blocked"),
+    (True, 90, 64, 32, 2, 2, 0, "blocked"),    # six of eight wavefronts unpack, fields of two bits
+    (False, 128, 64, 30, 4, 4, 0, "blocked"),
+    (False, 64, 64, 32, 2, 2, 0, "weed"),
 ])
 def test_chunks_that_share_the_unpacking(gpu, lloyd, d, Hq, T, k_bits, v_bits, sign, mapping):
     """A hundred rows and more per KV head over blocks enough for every workgroup to keep its tables and queries for a

@@ -5,13 +5,18 @@
 // matrix operands, into LDS (fp16, the operands in the order in which the matrix instructions take them: 32 KB per block at
 // head_dim 128, two blocks, one barrier per block), and every wavefront takes two tiles of sixteen rows against them, so that
 // an operand read from LDS serves both.  The matrix instructions (fp16 halves of queries and probabilities, as there) and the
-// softmax are what is left: 4096 and some 3500 cycles per SIMD for a block and 256 rows of 128, of 8900 that it takes -- matrix
-// and vector instructions of the two wavefronts of a SIMD overlap hardly at all, and at 128 with tables 180 bytes per lane of two tiles'
-// queries, sums, scores and probabilities go to scratch and back (256 registers are not enough; 20 bytes at 96 and with uniform cells).
+// softmax are what is left: 4096 and some 2800 cycles per SIMD for a block and 256 rows of 128, of 7200 that it takes -- unpacking
+// 1200, scores 1250, softmax 2100, values 1350 and the barrier, one after the other in both wavefronts of a SIMD.  What went (8900
+// cycles): loads dword by dword (request_narrow), reloads of spilled addresses (`anew`; instances of their own for up to four bits
+// a field), a masking and a subtraction per value in the split of the probabilities, the subtraction of the maximum per score, and
+// trips through LDS for the maxima.  64 positions x 32 heads on 8 of 128, K 3 + V 4 bits, 16 sequences of 4096 to 8192 tokens 266 ->
+// 235 us, of 8192 298 -> 264; of 4096, 4-bit cells 156 -> 143, 8-bit ones 175 -> 167.  (Half of the wavefronts half a block behind the
+// others, so that softmax and matrix instructions of a SIMD run beside each other: 226 us for 224 as it is, with three buffers of V;
+// unpacking between scores and softmax: 282, all of it scratch.)
 // The softmax, the split of the probabilities and the partials' write-out are those of kv_decode_mfma_kernel.h, for two tiles at a
 // time: a change to one is due in the other.
-// 64 positions x 32 heads on 8 of 128, K 3 + V 4 bits, 16 sequences: of 8192 tokens 360 -> 296 us, of 4096 205 -> 180, 4096 to 8192
-// 294 -> 257; 64 sequences of 1500, 5-bit fields 571 -> 379, 8-bit uniform ones 529 -> 341.  Where it is used: see kTilesToShare.
+// Beside the passes, before that: 16 sequences of 8192 tokens 360 -> 296 us, 4096 to 8192 294 -> 257; 64 sequences of 1500, 5-bit
+// fields 571 -> 379, 8-bit uniform ones 529 -> 341.  Where it is used: see kTilesToShare.
 // Against float64 its error is no larger (8192 tokens: Lloyd-Max 1.0e-6 against 1.1e-6, 8-bit cells 6e-6 against 10e-6).
 // Measured and dropped: one tile per wavefront (half the registers, twice the operand reads; 128 rows a workgroup: 132 rows 63 ->
 // 89 us, 32 rows 43 -> 49), that with a block's scores multiplied between the softmax of the block before and its products with V
@@ -23,6 +28,27 @@
 #include "kv_decode_mfma_kernel.h"
 
 namespace weedhip_mfma {
+
+// a less the fp16 value in h's low (high) half, exactly: one instruction (the compiler makes a conversion and a subtraction of it)
+__device__ __forceinline__ float less_low_half(float a, uint32_t h)
+{
+    float r;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(a));
+    return r;
+}
+__device__ __forceinline__ float less_high_half(float a, uint32_t h)
+{
+    float r;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(a));
+    return r;
+}
+
+// A lane's number anew: what is derived from it in a loop is computed there, not kept in (or spilled from) registers around it.
+__device__ __forceinline__ uint32_t anew(uint32_t lane)
+{
+    asm volatile("" : "+v"(lane));
+    return lane;
+}
 
 constexpr uint32_t kSharedWaves = 8;
 constexpr int kSharedTiles = 2; // tiles of sixteen rows per wavefront
@@ -67,7 +93,7 @@ template <int D> constexpr uint32_t shared_lds_bytes(uint32_t table_rows)
     return table_rows * kTableRowBytes + 2U * shared_block_bytes<D>() + 2U * 2U * 64U * 4U;
 }
 
-template <int D, bool LLOYD>
+template <int D, bool LLOYD, bool NARROW>
 __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaParams launch)
 {
     constexpr int QT = kSharedTiles, KS = D / 32, JB = D / 16;
@@ -95,7 +121,6 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
         const uint32_t w = p.table_image[i / 8];
         reinterpret_cast<uint4v *>(lds)[i] = uint4v{ w, w, w, w };
     }
-    const uint32_t vbase = (lane & 31) * 4, kbase = vbase + 128;
 
     const auto blk_off_at = [&](uint32_t i) { return p.uniform_blocks ? i * p.uniform_blocks : p.blk_off[i]; };
     uint32_t seq = 0;
@@ -139,7 +164,7 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
         float alpha = 0.0f;
         auto request_side = [&](const uint8_t *reg, uint32_t w, uint32_t blk, uint32_t (&x)[PER_WAVE][2]) __attribute__((always_inline)) {
             const uint32_t run = D * w / 32; // dwords per lane
-            const uint32_t *mine = reinterpret_cast<const uint32_t *>(reg + (uint64_t)blk * (8U * D * w)) + lane * run;
+            const uint32_t *mine = reinterpret_cast<const uint32_t *>(reg + (uint64_t)blk * (8U * D * w)) + anew(lane) * run;
 #pragma unroll
             for (int u = 0; u < PER_WAVE; ++u) {
                 const uint32_t i = wave + kSharedWaves * u;
@@ -148,53 +173,73 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
                 x[u][1] = mine[min(dw + 1, run - 1)];
             }
         };
+        // up to four bits a field: operands PER_WAVE wave .. PER_WAVE wave + PER_WAVE - 1, 64 bits from dword `first` of the run on in one load (a
+        // load per dword of operands eight apart was four times the lines asked for: 660 to 1100 cycles a block)
+        const auto first_dword = [&](uint32_t w) { return min((8 * w * PER_WAVE * wave) >> 5, D * w / 32 - 2); };
+        auto request_narrow = [&](const uint8_t *reg, uint32_t w, uint32_t blk, uint32_t (&x)[2]) __attribute__((always_inline)) {
+            typedef uint32_t uint2a __attribute__((ext_vector_type(2), aligned(4)));
+            const uint32_t mine = 4 * (anew(lane) * (D * w / 32) + first_dword(w));
+            const uint2a v = *reinterpret_cast<const uint2a *>(reg + (uint64_t)blk * (8U * D * w) + mine);
+            x[0] = v[0];
+            x[1] = v[1];
+        };
         auto request = [&](uint32_t blk) __attribute__((always_inline)) {
-            request_side(kreg, p.k.w, blk, kx);
-            request_side(vreg, p.v.w, blk, vx);
+            if constexpr (NARROW) {
+                request_narrow(kreg, p.k.w, blk, kx[0]);
+                request_narrow(vreg, p.v.w, blk, vx[0]);
+            } else {
+                request_side(kreg, p.k.w, blk, kx);
+                request_side(vreg, p.v.w, blk, vx);
+            }
             if constexpr (LLOYD) {
                 if (wave < 2) {
-                    alpha = alphas[blk * 64 + lane];
+                    alpha = alphas[blk * 64 + anew(lane)];
                 }
             }
         };
         auto unpack = [&](uint32_t blk, uint32_t buf) __attribute__((always_inline)) {
-            uint4v *to = reinterpret_cast<uint4v *>(operands + buf * shared_block_bytes<D>()) + lane;
-            auto side = [&](const uint8_t *reg, uint32_t w, const uint32_t (&x)[PER_WAVE][2], uint32_t lane_byte, uint32_t first) __attribute__((always_inline)) {
+            const uint32_t lane_ = anew(lane), vbase = (lane_ & 31) * 4, kbase = vbase + 128;
+            uint4v *k_to = reinterpret_cast<uint4v *>(operands + buf * shared_block_bytes<D>()) + lane_, *v_to = k_to + ITEMS * 64;
+            auto side = [&](const uint8_t *reg, uint32_t w, const uint32_t (&x)[PER_WAVE][2], uint32_t lane_byte, uint4v *to) __attribute__((always_inline)) {
                 const uint32_t run = D * w / 32;
-                const uint32_t *mine = reinterpret_cast<const uint32_t *>(reg + (uint64_t)blk * (8U * D * w)) + lane * run;
+                const uint32_t *mine = reinterpret_cast<const uint32_t *>(reg + (uint64_t)blk * (8U * D * w)) + lane_ * run;
 #pragma unroll
                 for (int u = 0; u < PER_WAVE; ++u) {
                     const uint32_t i = wave + kSharedWaves * u, bit = 8 * w * i;
                     if (i < (uint32_t)ITEMS) {
                         const half8 v = unpack_operand(w, x[u], mine + min((bit >> 5) + 2, run - 1), bit & 31, lane_byte);
-                        to[(first + i) * 64] = __builtin_bit_cast(uint4v, v);
+                        to[i * 64] = __builtin_bit_cast(uint4v, v);
                     }
                 }
             };
-            if (p.k.w <= 4 && p.v.w <= 4) {
+            if constexpr (NARROW) {
                 // (every lookup on its way before the first operand is put down)
                 uint4v r[2][PER_WAVE];
+                const auto cut = [&](uint32_t w, const uint32_t (&x)[2], int u, uint32_t lane_byte) __attribute__((always_inline)) {
+                    const uint32_t at = 8 * w * (PER_WAVE * wave + u) - 32 * first_dword(w);
+                    const uint32_t y[2] = { at < 32 ? x[0] : x[1], at < 32 ? x[1] : 0U };
+                    return lookup_operand(w, y, at & 31, lane_byte);
+                };
 #pragma unroll
                 for (int u = 0; u < PER_WAVE; ++u) {
-                    const uint32_t i = wave + kSharedWaves * u;
-                    r[0][u] = lookup_operand(p.k.w, kx[u], (8 * p.k.w * i) & 31, kbase);
-                    r[1][u] = lookup_operand(p.v.w, vx[u], (8 * p.v.w * i) & 31, vbase);
+                    r[0][u] = cut(p.k.w, kx[0], u, kbase);
+                    r[1][u] = cut(p.v.w, vx[0], u, vbase);
                 }
 #pragma unroll
                 for (int u = 0; u < PER_WAVE; ++u) {
-                    const uint32_t i = wave + kSharedWaves * u;
+                    const uint32_t i = PER_WAVE * wave + u;
                     if (i < (uint32_t)ITEMS) {
-                        to[i * 64] = r[0][u];
-                        to[(ITEMS + i) * 64] = r[1][u];
+                        k_to[i * 64] = r[0][u];
+                        v_to[i * 64] = r[1][u];
                     }
                 }
             } else {
-                side(kreg, p.k.w, kx, kbase, 0);
-                side(vreg, p.v.w, vx, vbase, ITEMS);
+                side(kreg, p.k.w, kx, kbase, k_to);
+                side(vreg, p.v.w, vx, vbase, v_to);
             }
             if constexpr (LLOYD) {
                 if (wave < 2) {
-                    scales[buf * 128 + wave * 64 + lane] = alpha;
+                    scales[buf * 128 + wave * 64 + lane_] = alpha;
                 }
             }
         };
@@ -240,10 +285,12 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
         }
         const float unscale = __uint_as_float((uint32_t)(127 - ep) << 23); // 2^-ep
         float m_run[QT], l_run[QT];
+        float shift[QT]; // what a score is moved by ahead of the exponential: beta q + ep - running maximum (0 while there is none)
         float4v O[QT][JB]; // lane (c, g), register r: row 4 g + r of the tile, coordinate 16 jb + c
 #pragma unroll
         for (int q = 0; q < QT; ++q) {
             m_run[q] = -INFINITY;
+            shift[q] = betaq[q] + (float)ep;
             l_run[q] = 0.0f;
 #pragma unroll
             for (int jb = 0; jb < JB; ++jb) {
@@ -251,47 +298,55 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
             }
         }
 
-        auto attend = [&](uint32_t blk, uint32_t buf) __attribute__((always_inline)) {
-            const uint4v *from = reinterpret_cast<const uint4v *>(operands + buf * shared_block_bytes<D>()) + lane;
-            const float4v *ak = reinterpret_cast<const float4v *>(scales + buf * 128) + g, *av = ak + 16;
-            // operands are read kAhead ahead of the matrix instructions that take them (K first, V behind it)
-            constexpr int kAhead = 3;
-            half8 ring[kAhead + 1];
+        // operands are read kAhead ahead of the matrix instructions that take them
+        constexpr int kAhead = 2, kRing = kAhead + 2;
+        half8 pa[QT][2][2]; // probabilities as A operands: [tile][half of the block][high, low]
+        float4v S[QT][4];
+        auto scores = [&](uint32_t buf) __attribute__((always_inline)) {
+            const uint4v *from = reinterpret_cast<const uint4v *>(operands + buf * shared_block_bytes<D>()) + anew(lane);
+            half8 ring[kRing];
             auto read = [&](auto ic) __attribute__((always_inline)) {
                 constexpr int i = decltype(ic)::value;
-                if constexpr (i < 2 * ITEMS) {
-                    ring[i % (kAhead + 1)] = __builtin_bit_cast(half8, from[i * 64]);
+                if constexpr (i < ITEMS) {
+                    ring[i % kRing] = __builtin_bit_cast(half8, from[((i % 4) * KS + i / 4) * 64]);
                 }
             };
             static_for<0, kAhead>(read);
-            float4v S[QT][4];
-            static_for<0, ITEMS>([&](auto ic) __attribute__((always_inline)) {
-                constexpr int i = decltype(ic)::value, t = i / KS, ks = i % KS;
+            // (operand i: tokens 16 (i % 4) .. + 15, coordinates 32 (i / 4) .. + 31; two at a time, so that a sum is next added to
+            // four instructions on)
+            static_for<0, ITEMS / 2>([&](auto ic) __attribute__((always_inline)) {
+                constexpr int i = 2 * decltype(ic)::value, t = i % 4, ks = i / 4;
                 read(std::integral_constant<int, i + kAhead>{});
+                read(std::integral_constant<int, i + 1 + kAhead>{});
                 __builtin_amdgcn_sched_barrier(0);
-                const half8 a = ring[i % (kAhead + 1)];
 #pragma unroll
-                for (int q = 0; q < QT; ++q) {
-                    if constexpr (ks == 0) {
-                        S[q][t] = float4v{ 0.0f, 0.0f, 0.0f, 0.0f };
+                for (int half = 0; half < 2; ++half) {
+#pragma unroll
+                    for (int n = 0; n < 2; ++n) {
+                        const half8 a = ring[(i + n) % kRing];
+#pragma unroll
+                        for (int q = 0; q < QT; ++q) {
+                            if (ks == 0 && half == 0) {
+                                S[q][t + n] = float4v{ 0.0f, 0.0f, 0.0f, 0.0f };
+                            }
+                            S[q][t + n] = mfma16(a, qop[q][half][ks], S[q][t + n]);
+                        }
                     }
-                    S[q][t] = mfma16(a, qop[q][0][ks], S[q][t]);
-                }
-#pragma unroll
-                for (int q = 0; q < QT; ++q) {
-                    S[q][t] = mfma16(a, qop[q][1][ks], S[q][t]);
                 }
             });
-            half8 pa[QT][2][2]; // probabilities as A operands: [tile][half of the block][high, low]
+        };
+        auto softmax = [&](uint32_t blk, uint32_t buf) __attribute__((always_inline)) {
+            const uint32_t g = anew(lane) >> 4;
+            const float4v *ak = reinterpret_cast<const float4v *>(scales + buf * 128) + g, *av = ak + 16;
 #pragma unroll
             for (int q = 0; q < QT; ++q) {
-                float C[4][4]; // token 16 t + 4 g + r, row c, in log2 units
+                float C[4][4]; // token 16 t + 4 g + r, row c, in log2 units above the running maximum, plus ep
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     const float4v k_scale = LLOYD ? ak[4 * t] : float4v{ p.k.alpha_const, p.k.alpha_const, p.k.alpha_const, p.k.alpha_const };
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        C[t][r] = fmaf(S[q][t][r], k_scale[r] * qscale[q], betaq[q]);
+                        C[t][r] = fmaf(S[q][t][r], k_scale[r] * qscale[q], shift[q]);
                     }
                 }
                 if (blk * 64 + 64 + hidden_max > L) {
@@ -314,8 +369,11 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
                     }
                 }
                 most = head_max<16>(most);
-                if (__any(most > m_run[q] + kSlack)) {
-                    const float m_new = fmaxf(m_run[q], most);
+                if (__any(most > (m_run[q] == -INFINITY ? -INFINITY : kSlack + (float)ep))) {
+                    // (a chunk's early positions can have a whole block hidden before anything was seen: still -inf)
+                    const float m_was = m_run[q] == -INFINITY ? 0.0f : m_run[q];
+                    const float m_new = fmaxf(m_run[q], most + (m_was - (float)ep));
+                    const float lower = m_was - (m_new == -INFINITY ? 0.0f : m_new);
                     const float scale = (m_run[q] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(m_run[q] - m_new);
                     l_run[q] *= scale;
                     float sr[4];
@@ -330,10 +388,16 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
                             O[q][jb][r] *= sr[r];
                         }
                     }
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            C[t][r] += lower;
+                        }
+                    }
                     m_run[q] = m_new;
+                    shift[q] += lower;
                 }
-                // (a chunk's early positions can have a whole block hidden before anything was seen: still -inf)
-                const float mm = (m_run[q] == -INFINITY ? 0.0f : m_run[q]) - (float)ep;
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
                     uint4v hi, lo;
@@ -344,36 +408,49 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
                         float pv[4];
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
-                            const float e = __builtin_amdgcn_exp2f(C[t][r] - mm); // exp2(-inf) = 0 masks the tail
+                            const float e = __builtin_amdgcn_exp2f(C[t][r]); // exp2(-inf) = 0 masks the tail
                             l_run[q] += e;
                             pv[r] = e * v_scale[r];
                         }
 #pragma unroll
                         for (int h2 = 0; h2 < 2; ++h2) {
-                            // hi = top 11 significant bits (exact in fp16), lo = the rest
+                            // hi = top 11 significant bits (fp16, towards zero), lo = the rest (exact, from hi as it came out)
                             const float a0 = pv[2 * h2], a1 = pv[2 * h2 + 1];
-                            const float h0 = __uint_as_float(__float_as_uint(a0) & 0xffffe000u);
-                            const float h1 = __uint_as_float(__float_as_uint(a1) & 0xffffe000u);
-                            hi[2 * half + h2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(h0, h1));
-                            lo[2 * half + h2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a0 - h0, a1 - h1));
+                            const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a0, a1));
+                            hi[2 * half + h2] = h;
+                            lo[2 * half + h2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(less_low_half(a0, h), less_high_half(a1, h)));
                         }
                     }
                     pa[q][u][0] = __builtin_bit_cast(half8, hi);
                     pa[q][u][1] = __builtin_bit_cast(half8, lo);
                 }
             }
-            static_for<0, ITEMS>([&](auto ic) __attribute__((always_inline)) {
-                constexpr int i = decltype(ic)::value, u = i / JB, jb = i % JB;
-                read(std::integral_constant<int, ITEMS + i + kAhead>{});
-                __builtin_amdgcn_sched_barrier(0);
-                const half8 b = ring[(ITEMS + i) % (kAhead + 1)];
-#pragma unroll
-                for (int q = 0; q < QT; ++q) {
-                    O[q][jb] = mfma16(pa[q][u][0], b, O[q][jb]);
+        };
+        auto values = [&](uint32_t buf) __attribute__((always_inline)) {
+            const uint4v *from = reinterpret_cast<const uint4v *>(operands + buf * shared_block_bytes<D>()) + ITEMS * 64 + anew(lane);
+            half8 ring[kRing];
+            auto read = [&](auto ic) __attribute__((always_inline)) {
+                constexpr int i = decltype(ic)::value;
+                if constexpr (i < ITEMS) {
+                    ring[i % kRing] = __builtin_bit_cast(half8, from[i * 64]);
                 }
+            };
+            static_for<0, kAhead>(read);
+            static_for<0, ITEMS / 2>([&](auto ic) __attribute__((always_inline)) {
+                constexpr int i = 2 * decltype(ic)::value, u = i / JB, jb = i % JB;
+                read(std::integral_constant<int, i + kAhead>{});
+                read(std::integral_constant<int, i + 1 + kAhead>{});
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int q = 0; q < QT; ++q) {
-                    O[q][jb] = mfma16(pa[q][u][1], b, O[q][jb]);
+                for (int half = 0; half < 2; ++half) {
+#pragma unroll
+                    for (int n = 0; n < 2; ++n) {
+                        const half8 b = ring[(i + n) % kRing];
+#pragma unroll
+                        for (int q = 0; q < QT; ++q) {
+                            O[q][jb + n] = mfma16(pa[q][u][half], b, O[q][jb + n]);
+                        }
+                    }
                 }
             });
         };
@@ -393,7 +470,9 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
                 request(min(blk + 2, b1 - 1));
             }
             if (works) {
-                attend(blk, buf);
+                scores(buf);
+                softmax(blk, buf);
+                values(buf);
             }
             __syncthreads();
         }
@@ -430,7 +509,7 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
     }
 }
 
-template <int D, bool LLOYD> int launch_shared(const MfmaParams &p, hipStream_t s)
+template <int D, bool LLOYD, bool NARROW> int launch_shared(const MfmaParams &p, hipStream_t s)
 {
     constexpr size_t most = shared_lds_bytes<D>(256);
     static_assert(most <= 160u * 1024u, "tables and blocks exceed a compute unit's LDS");
@@ -438,7 +517,7 @@ template <int D, bool LLOYD> int launch_shared(const MfmaParams &p, hipStream_t 
     static std::once_flag configured;
     static hipError_t config_status = hipSuccess;
     std::call_once(configured, [] {
-        config_status = hipFuncSetAttribute((const void *)decode_shared_kernel<D, LLOYD>,
+        config_status = hipFuncSetAttribute((const void *)decode_shared_kernel<D, LLOYD, NARROW>,
                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
     });
     WEED_HIP_CHECK(config_status);
@@ -448,14 +527,18 @@ template <int D, bool LLOYD> int launch_shared(const MfmaParams &p, hipStream_t 
     }
     const uint32_t units = (p.total_blocks + p.runs.unit_blocks - 1) / p.runs.unit_blocks;
     const uint32_t grid = (units + 7) / 8 * 8 * p.grid_passes;
-    decode_shared_kernel<D, LLOYD>
+    decode_shared_kernel<D, LLOYD, NARROW>
         <<<grid, 64 * kSharedWaves, shared_lds_bytes<D>(mfma_table_rows(p.k.w, p.v.w)), s>>>(p);
     WEED_HIP_LAUNCH_CHECK();
     return WEED_HIP_OK;
 }
 template <int D> int launch_shared_d(const MfmaParams &p, hipStream_t s)
 {
-    return p.k.alpha != nullptr ? launch_shared<D, true>(p, s) : launch_shared<D, false>(p, s);
+    const bool narrow = p.k.w <= 4 && p.v.w <= 4; // (their instances need none of the registers that the other widths' unpacking takes)
+    if (p.k.alpha != nullptr) {
+        return narrow ? launch_shared<D, true, true>(p, s) : launch_shared<D, true, false>(p, s);
+    }
+    return narrow ? launch_shared<D, false, true>(p, s) : launch_shared<D, false, false>(p, s);
 }
 
 } // namespace weedhip_mfma

@@ -234,6 +234,20 @@ template <int CTRL, int BANK_MASK> __device__ __forceinline__ float dpp_f32(floa
 }
 constexpr int kRowShl = 0x100, kRowShr = 0x110, kRowRor = 0x120;
 
+// Every lane's value beside that of the lane 16 (32) further on or back, in the order of the lanes: the swap instructions, which
+// take no trip through LDS.
+typedef uint32_t uint2r __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint2r rows_of_16(float v)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return uint2r{ (uint32_t)r[0], (uint32_t)r[1] };
+}
+__device__ __forceinline__ uint2r rows_of_32(float v)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return uint2r{ (uint32_t)r[0], (uint32_t)r[1] };
+}
+
 // Combine over the lanes that hold the same head: c % GP equal inside a row, then the 4 rows.
 template <int GP> __device__ __forceinline__ float head_max(float v)
 {
@@ -243,8 +257,10 @@ template <int GP> __device__ __forceinline__ float head_max(float v)
     if constexpr (GP <= 8) {
         v = fmaxf(v, dpp_f32<kRowRor + 8, 0xf>(v, v));
     }
-    v = fmaxf(v, __shfl_xor(v, 16));
-    return fmaxf(v, __shfl_xor(v, 32));
+    const uint2r r = rows_of_16(v);
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    const uint2r h = rows_of_32(v);
+    return fmaxf(__uint_as_float(h[0]), __uint_as_float(h[1]));
 }
 template <int GP> __device__ __forceinline__ float head_sum(float v)
 {
@@ -254,8 +270,10 @@ template <int GP> __device__ __forceinline__ float head_sum(float v)
     if constexpr (GP <= 8) {
         v += dpp_f32<kRowRor + 8, 0xf>(v, v);
     }
-    v += __shfl_xor(v, 16);
-    return v + __shfl_xor(v, 32);
+    const uint2r r = rows_of_16(v);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    const uint2r h = rows_of_32(v);
+    return __uint_as_float(h[0]) + __uint_as_float(h[1]);
 }
 
 // Query head that row `x` of this launch's tile stands for under KV head `kvh`: the launch covers the rows
