@@ -1273,3 +1273,26 @@ def test_matmul_batched_of_one_product_over_k_ranges(gpu, M, N, K, fp32_instruct
     # sums of integers below 2^24: exact in every order
     assert torch.equal(out[0, 0].double().cpu(), a[0, 0].double().cpu() @ b[0, 0].double().cpu())
     assert torch.all(out[:, 1:] == 7.0)
+
+
+@pytest.mark.parametrize("M,N,K", [(1024, 1024, 1040), (4096, 4096, 560), (512, 1024, 4112)])
+@pytest.mark.parametrize("kind", ["plain", "tiny", "infinite"])
+def test_large_whole_tiles_with_half_a_slice(gpu, M, N, K, kind):
+    """k a multiple of 16 but not of 32: exact where sums are integers below 2^24, scaled by powers of two or not, and an
+    infinity stays in its row."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+    A = torch.randint(-32, 33, (M, K), generator=gen, device="cuda").float()
+    B = torch.randint(-32, 33, (N, K), generator=gen, device="cuda").float().t()
+    want = A.double() @ B.double().contiguous()
+    if kind == "tiny":
+        A, B = A * 2.0 ** -119, B * 2.0 ** 119
+    elif kind == "infinite":
+        A[M // 3, K - 2] = float("inf")
+        want = A.double() @ B.double().contiguous()
+    C = torch.zeros((M, N), device="cuda")
+    torch.cuda.synchronize()
+    gpu.matmul(A, B, C)
+    gpu.sync()
+    assert torch.equal(torch.nan_to_num(C.double(), nan=0.5), torch.nan_to_num(want, nan=0.5))
