@@ -13,8 +13,9 @@
 // 235 us, of 8192 298 -> 264; of 4096, 4-bit cells 156 -> 143, 8-bit ones 175 -> 167.  (Half of the wavefronts half a block behind the
 // others, so that softmax and matrix instructions of a SIMD run beside each other: 226 us for 224 as it is, with three buffers of V;
 // unpacking between scores and softmax: 282, all of it scratch.)
-// The softmax, the split of the probabilities and the partials' write-out are those of kv_decode_mfma_kernel.h, for two tiles at a
-// time: a change to one is due in the other.
+// The partials' write-out is that of kv_decode_mfma_kernel.h for two tiles at a time: a change to one is due in the other.  The
+// softmax there subtracts the maximum and masks the probabilities' high halves in instructions of their own: as it is here, passes
+// gained 1 to 3 % and other calls lost 0.5 to 1 %.
 // Beside the passes, before that: 16 sequences of 8192 tokens 360 -> 296 us, 4096 to 8192 294 -> 257; 64 sequences of 1500, 5-bit
 // fields 571 -> 379, 8-bit uniform ones 529 -> 341.  Where it is used: see kTilesToShare.
 // Against float64 its error is no larger (8192 tokens: Lloyd-Max 1.0e-6 against 1.1e-6, 8-bit cells 6e-6 against 10e-6).
