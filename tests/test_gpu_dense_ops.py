@@ -1296,3 +1296,28 @@ def test_large_whole_tiles_with_half_a_slice(gpu, M, N, K, kind):
     gpu.matmul(A, B, C)
     gpu.sync()
     assert torch.equal(torch.nan_to_num(C.double(), nan=0.5), torch.nan_to_num(want, nan=0.5))
+
+
+@pytest.mark.parametrize("a_col,b_col", [(True, True), (False, True), (True, False), (False, False)])
+@pytest.mark.parametrize("M,N,K,rows,cols", [(1024, 1024, 1040, 1024, 1024), (4096, 4096, 560, 4096, 4096), (512, 1024, 4112, 512, 1024),
+                                             (128, 128, 272, 128, 128), (1000, 4100, 4112, 896, 3968)])
+def test_whole_tiles_with_half_a_slice_multiply_exactly(gpu, a_col, b_col, M, N, K, rows, cols):
+    """K an odd multiple of 16 in whole 128 x 128 tiles, and in those around which a ragged product has strips: the fp32
+    instruction, whose products are exact, so that a sum of one term is that product rounded once, bit for bit."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+    full = torch.randn((M, K), generator=gen, device="cuda")
+    take = torch.randint(0, K, (N,), generator=gen, device="cuda")
+    factor = torch.randn((N,), generator=gen, device="cuda")
+    sparse = torch.zeros((K, N), device="cuda")
+    sparse[take, torch.arange(N, device="cuda")] = factor
+    want = full[:, take] * factor
+    a = full.t().contiguous().t() if a_col else full
+    b = sparse.t().contiguous().t() if b_col else sparse
+    out = torch.zeros((N, M), device="cuda").t()
+    torch.cuda.synchronize()
+    gpu.matmul(a, b, out)
+    gpu.sync()
+    assert torch.equal(out[:rows, :cols], want[:rows, :cols])
+    assert bool(((out.double() - want.double()).abs() <= 2.0 ** -22 * want.double().abs()).all())
