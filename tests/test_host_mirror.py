@@ -52,3 +52,11 @@ def test_host_mirror_on_device():
     out = _run([])
     assert "0 failed" in out and "test_attention_lloydmax" in out and "test_qwen_decoder_layer_prefill_then_decode" in out
     assert "test_projections_side_by_side" in out
+
+
+@pytest.mark.gpu
+def test_products_without_memory_for_their_partial_results():
+    """Whole sums in place of k ranges from 2^30 multiply-adds on, WEED_HIP_ENOMEM below, and nothing left behind by either."""
+    binary = os.path.join(HERE, "host", "_build", "test_scratch_limit")
+    proc = subprocess.run([binary], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=100)
+    assert proc.returncode == 0 and "0 failed" in proc.stdout, proc.stdout[-4000:]

@@ -99,6 +99,10 @@ int fail(int code, const char *fmt, ...)
     vsnprintf(buf, sizeof(buf), fmt, ap);
     va_end(ap);
     g_last_error = buf;
+    if (code == WEED_HIP_ENOMEM) {
+        // the runtime keeps an allocation's failure until it is asked for: the next launch, a good one, would read it as its own
+        (void)hipGetLastError();
+    }
     return code;
 }
 
