@@ -1321,3 +1321,33 @@ def test_whole_tiles_with_half_a_slice_multiply_exactly(gpu, a_col, b_col, M, N,
     gpu.sync()
     assert torch.equal(out[:rows, :cols], want[:rows, :cols])
     assert bool(((out.double() - want.double()).abs() <= 2.0 ** -22 * want.double().abs()).all())
+
+
+@pytest.mark.parametrize("a_col,b_col,o_col", [(True, True, True), (True, False, False), (False, True, False), (False, False, True)])
+@pytest.mark.parametrize("M,N,K", [(3456, 3456, 96), (2304, 3840, 128), (3332, 2308, 64), (3332, 2308, 36), (3331, 2309, 63), (3331, 2309, 128),
+                                   (3331, 2309, 129), (65, 65665, 32)])
+def test_short_sums_of_more_tiles_than_two_to_a_compute_unit(gpu, a_col, b_col, o_col, M, N, K):
+    """513 to 810 tiles over up to 128 k, three workgroups to a compute unit, and over one more: whole tiles, checked loads, loads off
+    the 16-byte grid, one to four slices.  Sums of products of integers up to 64 are exact in every order; of normal values
+    they keep the bound of test_products_off_the_sixteen_byte_grid."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+
+    def matrix(rows, cols, col, whole):
+        shape = (cols, rows) if col else (rows, cols)
+        x = torch.randint(-64, 65, shape, generator=gen, device="cuda").float() if whole else torch.randn(shape, generator=gen, device="cuda")
+        return x.t() if col else x
+
+    for whole in (True, False):
+        A, B, C = matrix(M, K, a_col, whole), matrix(K, N, b_col, whole), matrix(M, N, o_col, whole)
+        bias = torch.randint(-64, 65, (N,), generator=gen, device="cuda").float()
+        torch.cuda.synchronize()
+        gpu.linear(A, B, bias, C) if whole else gpu.matmul(A, B, C)
+        gpu.sync()
+        want = A.double().contiguous() @ B.double().contiguous()
+        if whole:
+            assert torch.equal(C.double(), want + bias.double())
+        else:
+            scale = A.double().abs().contiguous() @ B.double().abs().contiguous()
+            assert float(((C.double() - want).abs() / scale).max()) <= 4 * 1.2e-7
