@@ -1060,6 +1060,48 @@ def test_chunks_that_share_the_unpacking(gpu, lloyd, d, Hq, T, k_bits, v_bits, s
     cache.close()
 
 
+@pytest.mark.parametrize("d,bits,width", [(64, 4, 1000.0), (64, 4, 300.0), (96, 6, 100.0)])
+def test_chunks_of_uniform_cells_whose_constant_part_outweighs_the_scores(gpu, d, bits, width):
+    """Queries of one sign over keys whose coordinates cancel in pairs: what the cells' lower end adds to every score of a row is
+    hundreds of times the scores' spread.  The values change their sign halfway, so that results are the small difference of
+    two halves' weights, which the runs of blocks that a row is cut into hold apart: whatever two runs do not take off their
+    scores alike is in them.  A score's own rounding, by at most some four units of its constant part's last place, averages over
+    thousands of tokens; a quarter of one such unit, times the values' mean, is allowed for what does not."""
+    import math
+    import torch
+    S, Hkv, Hq, T, L = 4, 8, 32, 64, 12000
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(d + bits)
+    cache = gpu.KVCache(gpu.KV_UNIFORM, S, Hkv, d, L, bits, bits)
+    cache.set_scales(1.6, 1.6)
+    half = torch.rand((S, Hkv, L, d // 2), generator=gen, device="cuda") * 2 - 1
+    k = torch.stack((half, -half), -1).reshape(S, Hkv, L, d).contiguous()
+    v = torch.rand((S, Hkv, L, d), generator=gen, device="cuda")
+    v[:, :, L // 2:] *= -1
+    q = (width + torch.randn((S, T, Hq, d), generator=gen, device="cuda") * min(1.0, width)).contiguous()
+    out = torch.full_like(q, float("nan"))
+    kd, vd = (torch.zeros((S, Hkv, L, d), device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    cache.encode_append(k, v, rotate=0)
+    cache.dequant(0, kd)
+    cache.dequant(1, vd)
+    cache.decode_attn_chunk(q, out, gqa_mapping=gpu.GQA_BLOCKED, flags=0)
+    gpu.sync()
+    seen = torch.arange(L, device="cuda")[None, :] <= (L - T + torch.arange(T, device="cuda"))[:, None]
+    worst = 0.0
+    for s in range(S):
+        for h in range(Hkv):
+            rows = q[s, :, 4 * h:4 * h + 4].double().permute(1, 0, 2)
+            scores = (rows.reshape(4 * T, d) @ kd[s, h].double().t().contiguous()).view(4, T, L) / math.sqrt(d)
+            weights = torch.softmax(scores.masked_fill(~seen, float("-inf")), -1)
+            want = (weights.view(4 * T, L) @ vd[s, h].double()).view(4, T, d)
+            worst = max(worst, float((out[s, :, 4 * h:4 * h + 4].double().permute(1, 0, 2) - want).abs().max()))
+    constant = 1.6 * width * d * math.log2(math.e) / math.sqrt(d)
+    unit = 2.0 ** (math.floor(math.log2(constant)) - 23)
+    assert worst <= 0.25 * math.log(2.0) * 0.5 * unit + 4e-6, (worst, unit)
+    cache.close()
+
+
 _PLANS = """
 import json, sys
 import torch

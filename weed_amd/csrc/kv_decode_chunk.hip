@@ -18,7 +18,10 @@
 // gained 1 to 3 % and other calls lost 0.5 to 1 %.
 // Beside the passes, before that: 16 sequences of 8192 tokens 360 -> 296 us, 4096 to 8192 294 -> 257; 64 sequences of 1500, 5-bit
 // fields 571 -> 379, 8-bit uniform ones 529 -> 341.  Where it is used: see kTilesToShare.
-// Against float64 its error is no larger (8192 tokens: Lloyd-Max 1.0e-6 against 1.1e-6, 8-bit cells 6e-6 against 10e-6).
+// Against float64 its error is no larger than the passes' (16 sequences of 4096 to 8192 tokens, of the result's norm: Lloyd-Max 5.5e-7
+// against 5.6e-7, 8-bit cells 6.3e-5 against 6.7e-5; queries of eight times the width 1.2e-6, 1.3e-6 and 3.5e-6, 3.6e-6).
+// At 128 with tables 52 bytes a lane of two tiles' queries, sums and scores still go to scratch and back, 108 where a field has more
+// than four bits; no other instance has any.
 // Measured and dropped: one tile per wavefront (half the registers, twice the operand reads; 128 rows a workgroup: 132 rows 63 ->
 // 89 us, 32 rows 43 -> 49), that with a block's scores multiplied between the softmax of the block before and its products with V
 // between the scores' arithmetic (16 sequences of 8192 tokens 345 us), and with two blocks' packed words on their way instead of
@@ -43,6 +46,9 @@ __device__ __forceinline__ float less_high_half(float a, uint32_t h)
     asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(a));
     return r;
 }
+
+typedef float float2p __attribute__((ext_vector_type(2)));
+typedef _Float16 half2p __attribute__((ext_vector_type(2)));
 
 // A lane's number anew: what is derived from it in a loop is computed there, not kept in (or spilled from) registers around it.
 __device__ __forceinline__ uint32_t anew(uint32_t lane)
@@ -248,7 +254,8 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
         // ---- this wavefront's rows: tiles QT wave .. QT wave + QT - 1 of sixteen; lane c of a tile's column works on row c ----
         const bool works = QT * 16 * wave < p.G;
         half8 qop[QT][2][KS];
-        float qscale[QT], betaq[QT];
+        float qscale[QT];
+        float m_first[QT]; // what stands for a row's running maximum while it has seen nothing
         uint32_t hidden[QT];
         const uint32_t hidden_max = p.q_tokens - 1U;
 #pragma unroll
@@ -268,7 +275,7 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
                 qop[q][1][ks] = __builtin_bit_cast(half8, lo);
             }
             qscale[q] = ok ? p.q_scale[row] : 0.0f;
-            betaq[q] = ok ? p.k.beta * p.q_sum[row] : 0.0f;
+            m_first[q] = (!LLOYD && ok) ? -__builtin_rintf(p.k.beta * p.q_sum[row]) : 0.0f;
             const uint32_t pair = p.head_first + hs; // index among the KV head's (position, head) pairs
             hidden[q] = (hidden_max && ok) ? hidden_max - (p.blocked ? pair % p.q_tokens : pair / p.real_group) : 0U;
         }
@@ -285,13 +292,17 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
             ep = ep > 100 ? 100 : (ep < -100 ? -100 : ep);
         }
         const float unscale = __uint_as_float((uint32_t)(127 - ep) << 23); // 2^-ep
+        // The running maximum of a row's scores, in whole log2 units: what a score is moved by, ep - m_run, what older sums are scaled
+        // by and what the merge scales partials by are exact then, so no two runs of a row differ in what they took off their
+        // scores.  (Taken as it was, off the sum of ep and what the uniform coder's constant part adds to every score of a row, it was
+        // rounded to that sum's size: queries of one sign and 100 normal values' width, 4-bit cells, errors 3.6e-5 -> 4.1e-5
+        // of the result's norm.  A softmax does not depend on that part; m_first takes it off a run's first scores, which are as
+        // large as it otherwise and rounded accordingly.)
         float m_run[QT], l_run[QT];
-        float shift[QT]; // what a score is moved by ahead of the exponential: beta q + ep - running maximum (0 while there is none)
         float4v O[QT][JB]; // lane (c, g), register r: row 4 g + r of the tile, coordinate 16 jb + c
 #pragma unroll
         for (int q = 0; q < QT; ++q) {
             m_run[q] = -INFINITY;
-            shift[q] = betaq[q] + (float)ep;
             l_run[q] = 0.0f;
 #pragma unroll
             for (int jb = 0; jb < JB; ++jb) {
@@ -341,13 +352,14 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
             const float4v *ak = reinterpret_cast<const float4v *>(scales + buf * 128) + g, *av = ak + 16;
 #pragma unroll
             for (int q = 0; q < QT; ++q) {
+                const float shift = (float)ep - (m_run[q] == -INFINITY ? m_first[q] : m_run[q]);
                 float C[4][4]; // token 16 t + 4 g + r, row c, in log2 units above the running maximum, plus ep
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     const float4v k_scale = LLOYD ? ak[4 * t] : float4v{ p.k.alpha_const, p.k.alpha_const, p.k.alpha_const, p.k.alpha_const };
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        C[t][r] = fmaf(S[q][t][r], k_scale[r] * qscale[q], shift[q]);
+                        C[t][r] = fmaf(S[q][t][r], k_scale[r] * qscale[q], shift);
                     }
                 }
                 if (blk * 64 + 64 + hidden_max > L) {
@@ -372,9 +384,9 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
                 most = head_max<16>(most);
                 if (__any(most > (m_run[q] == -INFINITY ? -INFINITY : kSlack + (float)ep))) {
                     // (a chunk's early positions can have a whole block hidden before anything was seen: still -inf)
-                    const float m_was = m_run[q] == -INFINITY ? 0.0f : m_run[q];
-                    const float m_new = fmaxf(m_run[q], most + (m_was - (float)ep));
-                    const float lower = m_was - (m_new == -INFINITY ? 0.0f : m_new);
+                    const float m_was = m_run[q] == -INFINITY ? m_first[q] : m_run[q];
+                    const float m_new = fmaxf(m_run[q], __builtin_ceilf(most + (m_was - (float)ep)));
+                    const float lower = m_new == -INFINITY ? 0.0f : m_was - m_new;
                     const float scale = (m_run[q] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(m_run[q] - m_new);
                     l_run[q] *= scale;
                     float sr[4];
@@ -397,7 +409,6 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
                         }
                     }
                     m_run[q] = m_new;
-                    shift[q] += lower;
                 }
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
@@ -415,11 +426,11 @@ __global__ void __launch_bounds__(64 * kSharedWaves) decode_shared_kernel(MfmaPa
                         }
 #pragma unroll
                         for (int h2 = 0; h2 < 2; ++h2) {
-                            // hi = top 11 significant bits (fp16, towards zero), lo = the rest (exact, from hi as it came out)
+                            // hi = top 11 significant bits (fp16, towards zero), lo = the rest (exact, from hi as it came out) to the nearest
                             const float a0 = pv[2 * h2], a1 = pv[2 * h2 + 1];
                             const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a0, a1));
                             hi[2 * half + h2] = h;
-                            lo[2 * half + h2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(less_low_half(a0, h), less_high_half(a1, h)));
+                            lo[2 * half + h2] = __builtin_bit_cast(uint32_t, __builtin_convertvector(float2p{ less_low_half(a0, h), less_high_half(a1, h) }, half2p));
                         }
                     }
                     pa[q][u][0] = __builtin_bit_cast(half8, hi);
