@@ -1112,10 +1112,15 @@ def test_products_with_long_strides(gpu, along_rows):
     assert float(((out.double() - a.double() @ b.double()).abs() / scale).max()) <= 4 * 1.2e-7
 
 
-@pytest.mark.parametrize("M,N,K", [(128, 128, 256), (256, 384, 1024), (130, 133, 260), (71, 515, 2051)])
+# Products in tiles of 256 x 256: whole ones, checked loads, loads off the 16-byte grid, k ranges with either (which ones they are
+# planned as: test_matmul_plan_cpu.py).
+LARGE_TILES = [(4096, 4096, 544), (4092, 4088, 548), (4093, 4087, 547), (1804, 5124, 3996), (1803, 5123, 3997)]
+
+
+@pytest.mark.parametrize("M,N,K", [(128, 128, 256), (256, 384, 1024), (130, 133, 260), (71, 515, 2051)] + LARGE_TILES)
 @pytest.mark.parametrize("mirrored", [False, True])
 def test_split_products_with_one_term_a_sum(gpu, M, N, K, mirrored):
-    """Sums of a single term, whole tiles, k ranges and sizes off the 16-byte grid: a column taken by a one is the column bit for
+    """Sums of a single term, whole tiles of either size, k ranges and sizes off the 16-byte grid: a column taken by a one is the column bit for
     bit, whatever the magnitudes beside it (2^-90 to 1: three exact parts lie in bfloat16's normal range); integers of 12 bits
     are multiplied exactly; and a product of two values errs by the products of parts that are left out, 2^-23 of it, and two
     roundings."""
@@ -1208,7 +1213,7 @@ def test_products_off_the_sixteen_byte_grid_of_tiny_values_that_meet_zeros(gpu, 
 @pytest.mark.parametrize("batch,M,N,K", [(1, 1156, 132, 64), (1, 132, 1156, 40), (3, 1028, 260, 36), (1, 1285, 517, 33), (1, 264, 132, 2052),
                                          (5, 129, 131, 95)])
 def test_split_products_tile_order(gpu, batch, M, N, K):
-    """More tiles of rows than a band holds, fewer tiles than XCDs, k ranges and products of a batch: every tile exactly once.
+    """Grids in their own order (fewer than 512 workgroups), k ranges and products of a batch: every tile exactly once.
 
     Products of integers up to 64 over these k are exact in every order, so nothing but a wrong tile can differ."""
     import torch
@@ -1223,9 +1228,69 @@ def test_split_products_tile_order(gpu, batch, M, N, K):
     assert torch.equal(C[0].cpu().double(), want)
 
 
+# 512 workgroups and more, which are placed by XCD: remainders modulo 8, short last bands, products of a batch and k ranges whose
+# workgroups cross from one XCD's run into the next, and both tiles (see test_matmul_plan_cpu.py).
+PLACED = [(1, 3332, 2308, 64), (7, 1028, 1028, 36), (7, 1028, 1028, 132), (5, 1541, 1157, 33), (1, 3341, 2350, 516), (1, 4494, 540, 2052),
+          (1, 5262, 7869, 516), (1, 3474, 2549, 2500)]
+
+
+@pytest.mark.parametrize("batch,M,N,K", PLACED)
+def test_split_products_placed_by_xcd(gpu, batch, M, N, K):
+    """Every tile of every product and range exactly once: sums of products of integers up to 64 over these k stay below 2^24, exact in
+    every order, so nothing but a wrong tile can differ."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+    A = torch.randint(-64, 65, (1, batch, M, K), generator=gen, device="cuda").float()
+    B = torch.randint(-64, 65, (1, batch, N, K), generator=gen, device="cuda").float().transpose(2, 3)
+    C = torch.full((1, batch, M, N), 7.5, device="cuda")
+    torch.cuda.synchronize()
+    gpu.matmul_batched(A, B, C) if batch > 1 else gpu.matmul(A[0, 0], B[0, 0], C[0, 0])
+    gpu.sync()
+    for a, b, c in zip(A[0], B[0], C[0]):
+        assert torch.equal(c.double(), a.double() @ b.double().contiguous())
+
+
 @pytest.mark.parametrize("a_col,b_col,o_col", [(True, True, True), (True, False, False), (False, True, False), (False, False, True)])
-@pytest.mark.parametrize("M,N,K,infinite", [(4096, 4096, 544, False), (4092, 4088, 548, False), (4093, 4087, 547, False), (4093, 4087, 547, True),
-                                            (1804, 5124, 3996, False), (1803, 5123, 3997, False)])
+@pytest.mark.parametrize("M,N,K", LARGE_TILES)
+@pytest.mark.parametrize("wide_range", [False, True])
+def test_split_products_in_large_tiles_keep_fp32_accuracy(gpu, a_col, b_col, o_col, M, N, K, wide_range):
+    """Tiles of 256 x 256 by values that take all three parts of the split: the bounds of test_matmul_split_products_keep_fp32_accuracy,
+    against float64 and beside the fp32 instruction."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K + wide_range)
+
+    def matrix(rows, cols, col):
+        x = torch.randn((cols, rows) if col else (rows, cols), generator=gen, device="cuda")
+        if wide_range:
+            x *= torch.exp2(torch.randint(-20, 21, x.shape, generator=gen, device="cuda").float())
+        return x.t() if col else x
+
+    A, B, C = matrix(M, K, a_col), matrix(K, N, b_col), matrix(M, N, o_col)
+    want = A.double().contiguous() @ B.double().contiguous()
+    scale = A.double().abs().contiguous() @ B.double().abs().contiguous()
+    worst, mean = {}, {}
+    for fp32_instruction in (True, False):
+        torch.cuda.synchronize()
+        gpu.matmul_tuning(fp32_instruction)
+        try:
+            gpu.matmul(A, B, C)
+        finally:
+            gpu.matmul_tuning(False)
+        gpu.sync()
+        err = (C.double() - want).abs() / scale
+        worst[fp32_instruction], mean[fp32_instruction] = float(err.max()), float(err.mean())
+    # the yardstick itself is sane: K / 2 roundings of a running sum below `scale`, each within 2^-24 of it and evenly spread, make
+    # sqrt(K / 6) 2^-24 in the root mean square, and 10^7 such values reach 5.3 times that
+    assert worst[True] <= 5.3 * (K / 6) ** 0.5 * 2.0 ** -24, worst
+    assert worst[False] <= 1.5 * worst[True] + 5e-8, (worst, mean)
+    assert mean[False] <= 1.25 * mean[True], (worst, mean)
+
+
+@pytest.mark.parametrize("a_col,b_col,o_col", [(True, True, True), (True, False, False), (False, True, False), (False, False, True)])
+@pytest.mark.parametrize("M,N,K,infinite", [shape + (False,) for shape in LARGE_TILES] + [(4093, 4087, 547, True), (1803, 5123, 3997, True),
+                                                                                          (2709, 921, 1501, True)])
 def test_split_products_in_large_tiles(gpu, a_col, b_col, o_col, M, N, K, infinite):
     """Whole tiles of 256, checked loads, loads off the 16-byte grid, k ranges.
 
@@ -1323,9 +1388,12 @@ def test_whole_tiles_with_half_a_slice_multiply_exactly(gpu, a_col, b_col, M, N,
     assert bool(((out.double() - want.double()).abs() <= 2.0 ** -22 * want.double().abs()).all())
 
 
+# More tiles than two to a compute unit over up to 128 k (see test_matmul_plan_cpu.py)
+SHORT_SUMS = [(3456, 3456, 96), (2304, 3840, 128), (3332, 2308, 64), (3332, 2308, 36), (3331, 2309, 63), (3331, 2309, 128), (65, 65665, 32)]
+
+
 @pytest.mark.parametrize("a_col,b_col,o_col", [(True, True, True), (True, False, False), (False, True, False), (False, False, True)])
-@pytest.mark.parametrize("M,N,K", [(3456, 3456, 96), (2304, 3840, 128), (3332, 2308, 64), (3332, 2308, 36), (3331, 2309, 63), (3331, 2309, 128),
-                                   (3331, 2309, 129), (65, 65665, 32)])
+@pytest.mark.parametrize("M,N,K", SHORT_SUMS + [(3331, 2309, 129)])
 def test_short_sums_of_more_tiles_than_two_to_a_compute_unit(gpu, a_col, b_col, o_col, M, N, K):
     """513 to 810 tiles over up to 128 k, three workgroups to a compute unit, and over one more: whole tiles, checked loads, loads off
     the 16-byte grid, one to four slices.  Sums of products of integers up to 64 are exact in every order; of normal values

@@ -266,3 +266,46 @@ def test_products_in_a_graph_outlive_the_scratch_they_were_captured_with(gpu, wa
         gpu.sync()
         for (M, N, K), (_, _, out, want, bound) in zip(shapes, work):
             assert bool(((out.double() - want).abs() <= bound).all()), (M, N, K, i)
+
+
+# Captured products of 2^30 multiply-adds and more: k ranges of either tile, on and off the 16-byte grid, strips, and whole tiles of 256,
+# with what of the scratch that SCRATCH_BEFORE leaves they find room for (see test_matmul_plan_cpu.py).
+LARGE_IN_A_GRAPH = [(512, 4096, 4096), (2708, 920, 1500), (1001, 4096, 4096), (1030, 4096, 4096), (4096, 4096, 544)]
+SCRATCH_BEFORE = (640, 1024, 4096)
+
+
+@pytest.mark.parametrize("scratch", ["none", "some", "all"])
+def test_large_products_in_a_graph_keep_to_the_scratch_they_find(gpu, scratch):
+    """Captured before the library has any scratch, with less of it than their plans ask for, and with all of it: right on every
+    replay, also after eager calls that took a larger one."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(78)
+    gpu.shutdown()
+    gpu.check(gpu.load().weed_hip_init(0))
+    gpu.use_torch_stream(torch.cuda.current_stream())
+
+    def product(M, N, K):
+        a = torch.randn((K, M), generator=gen, device="cuda").t()
+        b = torch.randn((N, K), generator=gen, device="cuda").t()
+        return a, b, torch.zeros((N, M), device="cuda").t()
+
+    work = [product(*shape) for shape in LARGE_IN_A_GRAPH]
+    before, beside = product(*SCRATCH_BEFORE), product(1024, 2048, 8192)
+    for a, b, out in work if scratch == "all" else [before] if scratch == "some" else []:
+        gpu.matmul(a, b, out)
+    gpu.sync()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.current_stream()):
+        for a, b, out in work:
+            gpu.matmul(a, b, out)
+    wants = [(a.double().contiguous() @ b.double().contiguous(), a.double().abs().contiguous() @ b.double().abs().contiguous()) for a, b, _ in work]
+    for i in range(4):
+        for _, _, out in work:
+            out.fill_(float("nan"))
+        graph.replay()
+        gpu.sync()
+        for shape, (_, _, out), (want, scale) in zip(LARGE_IN_A_GRAPH, work, wants):
+            assert float(((out.double() - want).abs() / scale).max()) <= 4 * 1.2e-7, (shape, i)  # as the dense products' tests
+        gpu.matmul(*beside)
+        gpu.sync()
