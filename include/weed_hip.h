@@ -92,7 +92,8 @@ int weed_hip_matmul_f32(uint32_t M, uint32_t N, uint32_t K, const float *a_dev, 
 /* Which matrix instruction the large products run on (no counterpart in the reference; process-wide, takes effect
  * with the next call).  0, the default: products of at least 17 rows and columns whose operands are contiguous along
  * one dimension (of 17 to 64 rows against a k-contiguous weight with 256 k or more: those of 512 columns or more, and
- * off the 16-byte grid those of a k too long for the streaming kernel) run on the bfloat16 instruction with both
+ * off the 16-byte grid those of a k too long for the streaming kernel; whole tiles of 128 x 128 over a k that is a
+ * multiple of 16 but not of 32 excepted, which the fp32 instruction takes) run on the bfloat16 instruction with both
  * operands split exactly into three bfloat16 parts and six of the nine products of parts accumulated in fp32 -- 1.5
  * times the fp32 instruction's speed and more.  The error against the exact product is the fp32 instruction's own:
  * relative to sum_k |a_ik| |b_kj| per element, at k = 1028 over operands spanning 2^-20 .. 2^20, largest 7.1e-7

@@ -85,7 +85,10 @@ inline uint32_t choose_k_splits(uint64_t out_tiles, uint32_t K)
 // what its workgroups take in microseconds.  A round of 512 tiles of 128 x 128 (two workgroups per compute unit; up to 256 of them
 // take 0.8 of a round) or of 256 tiles of 256 x 256 takes so much per k and something for its start and write-out; partial sums
 // are written, read and added at 3.6 GB per millisecond.  The rates are a least-squares fit to 65 products of 65 to 4096 rows in up
-// to eleven splits each, which it meets within 5 %; `off_grid` is GUARD 2, whose loads and magnitudes cost a little more.
+// to eleven splits each; `off_grid` is GUARD 2, whose loads and magnitudes cost a little more.  Of 49 products drawn afterwards it is
+// within 5 % for 38 and within 10 % for 48 (1994 x 1088 x 896 takes 37 us for 44), and what it chooses is within 3 % of the fastest
+// tile and ranges in all but 1051 x 512 x 3136 off the grid (43.4 us whole, 37.4 in two ranges), 3324 x 2496 x 5248 (528, 500 in
+// three) and 2221 x 12800 x 1088 (370 in three, 358 in six).
 // Beside the rule for 128 x 128 tiles alone that stood here, which counted rounds of 256 and left more than 512 tiles whole: 1649 x
 // 5632 x 5824 851 -> 595 us, 556 x 5075 x 13240 788 -> 528, 1906 x 13504 x 9344 3198 -> 2432, 2036 x 1280 x 1984 80 -> 68,
 // 2364 x 689 x 1269 58 -> 46, 4096^3 632 -> 572.
@@ -98,7 +101,7 @@ inline TilePlan plan_tiles(uint32_t M, uint32_t N, uint32_t K, uint32_t batch, u
 {
     TilePlan best{ kTile, 1, 0, 0.0 };
     for (uint32_t tile : { kTile, kBig }) {
-        // (256 x 256: not for short sums, which are all write-out; 8000 x 128 x 2000, eight products: 258 and 278 us)
+        // (256 x 256: not for short sums, which are all write-out; 8000 x 128 x 2000, eight products: 238 and 278 us)
         if (tile == kBig && K < 512) {
             break;
         }
